@@ -12,12 +12,13 @@
 // dealt to the XCDs round-robin).  Each workgroup computes the prefix sums of
 // the batch itself (into LDS) and walks its range; a range may cut sequences,
 // whose pieces write fp32 partials (unnormalised O, running max in log2
-// units, sum).  A workgroup's range can end at most one cut sequence (a cut
-// sequence ending inside a range began before it, i.e. at the range's start),
-// so each workgroup leaves a 16-byte descriptor of that sequence (or none;
-// a plan instead holds one per sequence when sequences are fewer than
+// units, sum).  A workgroup's range can continue at most one cut sequence (it
+// began before the range, so it holds the range's start), so each workgroup
+// leaves a 16-byte merge descriptor (or none; a plan instead holds one per
+// sequence, and some to help with long ones, when sequences are fewer than
 // workgroups), and a second kernel, one workgroup per descriptor and kv head,
-// merges its pieces with log-sum-exp weights.  A sequence held by one workgroup is
+// merges its pieces with log-sum-exp weights: up to kMergeAlone pieces by one
+// workgroup, more by several.  A sequence held by one workgroup is
 // normalised and written directly.  (Merging in the main kernel by the last
 // piece to arrive measured slower every way it was built: with device-scope
 // release fences, which write back the XCD's L2, 2x; with write-through
@@ -162,7 +163,7 @@ struct AttnArgs {
   int32_t max_seq_len;  // host bound; longer device lengths are clamped to it
   uint16_t* out;
   int64_t out_bstride;  // elements
-  int4* desc;           // [n_wg] cut sequence ending in each workgroup: (b, grp, w0, npieces)
+  int4* desc;           // merge descriptors (see merge_desc)
   float* part_o;        // [slots][hpg][D]
   float2* part_ml;      // [slots][hpg] (running max in log2 units, sum)
   uint32_t ml_bytes, o_bytes;  // sizes of the two partial regions (< 2^31)
@@ -190,13 +191,43 @@ struct AttnArgs {
   int32_t n_desc;                      // merge descriptors (the combine grid's width)
 };
 
-// A plan indexes the merge descriptors by (kv-head group, sequence) when there
-// are fewer of those than workgroups, so that the combine grid has one
-// workgroup per sequence instead of one per main-kernel workgroup (the
-// Yi-1.5-9B batch: 64 against 256, of which 61 cut); otherwise, and without a
-// plan, by the workgroup holding the sequence's last piece.
+// A sequence of up to kMergeAlone pieces is merged by one workgroup per kv
+// head, in rounds of loads of all its items; one of more pieces by several,
+// each taking some of the items (a 131001-token sequence over 256 workgroups:
+// 26.3 us per layer by one workgroup per kv
+// head in 22 rounds of loads, 4.1 us shared).
+constexpr int kMergeAlone = 24;
+constexpr int kMaxHelpers = 64;  // workgroups (per kv head) that share one merge
+
+// Merge descriptor: sequence b of kv-head group grp, cut into np pieces held
+// by workgroups w0 .. w0 + np - 1; this descriptor's workgroup is number k of
+// the nh that merge it.  (np <= 2^15; b < 0: nothing to do.)
+__device__ __forceinline__ int4 merge_desc(int b, int grp, int w0, int np, int k, int nh) {
+  return make_int4(b, grp, w0 | (k << 16) | (nh << 23), np);
+}
+__device__ __forceinline__ int4 no_merge() { return make_int4(-1, 0, 0, 0); }
+// The descriptor of workgroup w, whose range starts in sequence b of group
+// grp held by workgroups [w0, w1]: the last of them merges a short cut
+// sequence, the ones after the first share a long one's merge.
+__device__ __forceinline__ int4 continued_desc(int b, int grp, int64_t w0, int64_t w1, int64_t w) {
+  const int np = (int)(w1 - w0 + 1);
+  if (np < 2 || w <= w0 || w > w1) return no_merge();
+  if (np <= kMergeAlone) return w == w1 ? merge_desc(b, grp, (int)w0, np, 0, 1) : no_merge();
+  const int k = (int)(w - w0 - 1), nh = min(np - 1, kMaxHelpers);
+  return k < nh ? merge_desc(b, grp, (int)w0, np, k, nh) : no_merge();
+}
+
+// A plan indexes the merge descriptors by (kv-head group, sequence) when
+// those, with kPlanHelpers to share the merges of long sequences, are no more
+// than the workgroups, so that the combine grid is that much smaller (the
+// Qwen2.5-7B heads, 128 sequences: 160 descriptors against 256, 0.8 us per layer);
+// otherwise, and without a plan, by the workgroup that continues the sequence.
+constexpr int kPlanHelpers = 32;
+// Long sequences of one launch: each takes more than kMergeAlone - 1 workgroups
+// beyond its first, and a workgroup continues at most one sequence.
+constexpr int kMaxLong = kMaxWorkgroups / kMergeAlone + 1;
 inline bool desc_per_sequence(int64_t batch, int64_t n_groups, int64_t n_wg) {
-  return batch * n_groups < n_wg;
+  return batch * n_groups + kPlanHelpers <= n_wg;
 }
 
 // Decode plan, in one device buffer: per main-kernel workgroup a record of 8
@@ -993,7 +1024,7 @@ paged_decode_attention_kernel(AttnArgs a) {
   // that every range is non-empty.
   const int64_t n_act = min((int64_t)a.n_wg, total);
   if ((int64_t)blockIdx.x >= n_act) {
-    if (tid == 0) a.desc[blockIdx.x] = make_int4(-1, 0, 0, 0);
+    if (tid == 0) a.desc[blockIdx.x] = no_merge();
     return;
   }
   int64_t P = div_floor((int64_t)blockIdx.x * total, n_act);
@@ -1024,14 +1055,12 @@ paged_decode_attention_kernel(AttnArgs a) {
     const int i0 = items_before(b0, p0);
     const int i1 = p1 == (int)W ? s_bcum[a.batch] : items_before(s_find[1], p1);
     if (first_pass) {
-      // The range's first piece is the only one that can end a cut sequence:
-      // describe it for the merge when it does.
+      // The range's first piece is the only one that can continue a cut
+      // sequence: describe it for the merge when it does.
       const int64_t w0 = owner_of(pbase + s_cum[b0] + kSegmentCost, total, n_act);
       const int64_t w1 = owner_of(pbase + s_cum[b0 + 1] - 1, total, n_act);
       if (tid == 0)
-        a.desc[blockIdx.x] = (w0 != w1 && w1 == (int64_t)blockIdx.x)
-                                 ? make_int4(b0, grp, (int)w0, (int)(w1 - w0 + 1))
-                                 : make_int4(-1, 0, 0, 0);
+        a.desc[blockIdx.x] = continued_desc(b0, grp, w0, w1, (int64_t)blockIdx.x);
       first_pass = false;
     }
     if (i1 > i0)
@@ -1051,7 +1080,7 @@ struct PlanArgs {
   int32_t max_seq_len;
   int32_t n_groups;
   int32_t n_wg;
-  int32_t desc_per_seq;  // desc indexed by grp * batch + b (else by workgroup)
+  int32_t desc_per_seq;  // descriptors indexed by grp * batch + b (else by workgroup)
   int32_t* wg;
   int4* desc;
   int32_t* first;
@@ -1105,7 +1134,7 @@ __global__ __launch_bounds__(64 * kHeadsPerGroup) void decode_plan_kernel(PlanAr
     int32_t* rec = p.wg + (int64_t)w * kPlanRecord;
     if (w >= n_act) {
       rec[0] = -1;
-      if (!p.desc_per_seq) p.desc[w] = make_int4(-1, 0, 0, 0);
+      if (!p.desc_per_seq) p.desc[w] = no_merge();
       continue;
     }
     const Range r = range_of(w);
@@ -1118,24 +1147,48 @@ __global__ __launch_bounds__(64 * kHeadsPerGroup) void decode_plan_kernel(PlanAr
     rec[6] = 0;
     rec[7] = 0;
     if (p.desc_per_seq) continue;
-    // the range's first piece is the only one that can end a cut sequence
+    // the range's first piece is the only one that can continue a cut sequence
     const int64_t pbase = (int64_t)r.gf * W;
     const int64_t w0 = owner_of(pbase + s_cum[r.b0] + kSegmentCost, total, n_act);
     const int64_t w1 = owner_of(pbase + s_cum[r.b0 + 1] - 1, total, n_act);
-    p.desc[w] = (w0 != w1 && w1 == (int64_t)w) ? make_int4(r.b0, r.gf, (int)w0, (int)(w1 - w0 + 1))
-                                               : make_int4(-1, 0, 0, 0);
+    p.desc[w] = continued_desc(r.b0, r.gf, w0, w1, w);
   }
-  if (p.desc_per_seq) {  // one descriptor per (group, sequence): cut or not
-    for (int e = gtid; e < p.n_groups * p.batch; e += gsz) {
+  // one descriptor per (group, sequence), then kPlanHelpers dealt over the
+  // long sequences (written by one workgroup: they share a count)
+  if (p.desc_per_seq && blockIdx.x == 0) {
+    __shared__ int32_t s_nlong;
+    __shared__ int4 s_long[kMaxLong];
+    const int n = p.n_groups * p.batch;
+    if (threadIdx.x == 0) s_nlong = 0;
+    __syncthreads();
+    for (int e = threadIdx.x; e < n; e += blockDim.x) {
       const int grp = e / p.batch, b = e % p.batch;
-      int4 d = make_int4(-1, 0, 0, 0);
+      int4 d = no_merge();
       if (s_bcum[b + 1] > s_bcum[b]) {
         const int64_t pbase = (int64_t)grp * W;
-        const int64_t w0 = owner_of(pbase + s_cum[b] + kSegmentCost, total, n_act);
-        const int64_t w1 = owner_of(pbase + s_cum[b + 1] - 1, total, n_act);
-        if (w0 != w1) d = make_int4(b, grp, (int)w0, (int)(w1 - w0 + 1));
+        const int w0 = (int)owner_of(pbase + s_cum[b] + kSegmentCost, total, n_act);
+        const int np = (int)owner_of(pbase + s_cum[b + 1] - 1, total, n_act) - w0 + 1;
+        if (np > kMergeAlone) {  // fewer than kMaxLong such sequences
+          s_long[atomicAdd(&s_nlong, 1)] = make_int4(e, w0, np, 0);
+          continue;
+        }
+        if (np > 1) d = merge_desc(b, grp, w0, np, 0, 1);
       }
       p.desc[e] = d;
+    }
+    __syncthreads();
+    const int R = s_nlong;
+    for (int x = threadIdx.x; x < R + kPlanHelpers; x += blockDim.x) {
+      // long sequence x itself, or helper i, which is number 1 + i / R of its
+      const int i = x - R, r = R == 0 ? 0 : i < 0 ? x : i % R;
+      const int at = i < 0 ? s_long[r].x : n + i;
+      int4 d = no_merge();
+      if (R > 0) {
+        const int4 l = s_long[r];
+        const int nh = 1 + (kPlanHelpers - r + R - 1) / R;
+        d = merge_desc(l.x % p.batch, l.x / p.batch, l.y, l.z, i < 0 ? 0 : 1 + i / R, nh);
+      }
+      p.desc[at] = d;
     }
   }
   auto id_of = [&](int i) -> int32_t {
@@ -1238,6 +1291,99 @@ __device__ __forceinline__ int64_t new_row_chunks(const AttnArgs& a) {
 }
 
 
+// The merge of a sequence of more than kMergeAlone pieces: the nh workgroups
+// (of one kv head) take runs of kMergeCols float4 columns (one 128-byte line of
+// a piece) in turn; the workgroup's 32 slices of 8 threads take every 32nd
+// piece each and meet through shuffles and LDS.  The sums' order does not
+// depend on nh, so every launch form gives the same bits.
+constexpr int kMergeCols = 8;
+constexpr int kMergeSlices = 64 * kHeadsPerGroup / kMergeCols;
+constexpr int kMergeAhead = 8;  // pieces a thread loads at once
+struct MergeState {
+  float m, l;
+  f32x4 o;
+  __device__ __forceinline__ void add(float m2, float l2, f32x4 o2) {
+    const float mn = fmaxf(m, m2);
+    // a side with no readable block: weight 0
+    const float w1 = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - mn);
+    const float w2 = m2 == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m2 - mn);
+    m = mn;
+    l = l * w1 + l2 * w2;
+    o = o * w1 + o2 * w2;
+  }
+};
+template <int DT, int D>
+__device__ __forceinline__ void merge_pieces_shared(const AttnArgs& a, const int4 d,
+                                                    MergeState (*s_m)[kMergeCols]) {
+  using E = Elem<DT>;
+  constexpr int D4 = D / 4;
+  const int b = d.x, grp = d.y, npieces = d.w;
+  const int h = grp * kHeadsPerGroup + blockIdx.y;
+  if (h >= a.n_kv_heads) return;
+  const int w0 = d.z & 0xffff, nh = (int)((uint32_t)d.z >> 23);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int sl = (int)threadIdx.x / kMergeCols;
+  const int64_t slot0 = (int64_t)w0 + (int64_t)grp * a.batch + b;
+  const auto mlr = byte_range(reinterpret_cast<const uint8_t*>(a.part_ml), a.ml_bytes);
+  const auto por = byte_range(reinterpret_cast<const uint8_t*>(a.part_o), a.o_bytes);
+  const uint32_t ml_step = (uint32_t)a.hpg * 8u, o_step = (uint32_t)a.hpg * D * 4u;
+  for (int c = (d.z >> 16) & 0x7f; c < a.group * D4 / kMergeCols; c += nh) {
+    const int it = kMergeCols * c + (int)threadIdx.x % kMergeCols;
+    const int64_t pidx0 = slot0 * a.hpg + blockIdx.y * a.group + it / D4;
+    const int col = 4 * (it % D4);
+    const uint32_t ml_off = (uint32_t)(pidx0 * 8), o_off = (uint32_t)((pidx0 * D + col) * 4);
+    MergeState st{-INFINITY, 0.f, f32x4{0.f, 0.f, 0.f, 0.f}};
+    for (int s0 = sl; s0 < npieces; s0 += kMergeAhead * kMergeSlices) {
+      float2 ml[kMergeAhead];
+      f32x4 po[kMergeAhead];
+#pragma unroll
+      for (int u = 0; u < kMergeAhead; ++u) {
+        const int s = s0 + u * kMergeSlices;
+        const bool ok = s < npieces;  // else past the ranges: zeros, no access
+        const u32x2 mw = __builtin_amdgcn_raw_buffer_load_b64(
+            mlr, ok ? ml_off + (uint32_t)s * ml_step : kPastRange, 0, 0);
+        const u32x4 ow = __builtin_amdgcn_raw_buffer_load_b128(
+            por, ok ? o_off + (uint32_t)s * o_step : kPastRange, 0, 0);
+        ml[u] = make_float2(ok ? __uint_as_float(mw.x) : -INFINITY, __uint_as_float(mw.y));
+        po[u] = f32x4{__uint_as_float(ow.x), __uint_as_float(ow.y), __uint_as_float(ow.z),
+                      __uint_as_float(ow.w)};
+      }
+      float mn = -INFINITY, lt = 0.f;
+#pragma unroll
+      for (int u = 0; u < kMergeAhead; ++u) mn = fmaxf(mn, ml[u].x);
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int u = 0; u < kMergeAhead; ++u) {
+        const float w = ml[u].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ml[u].x - mn);
+        o += po[u] * w;
+        lt += ml[u].y * w;
+      }
+      st.add(mn, lt, o);
+    }
+#pragma unroll
+    for (int x = kMergeCols; x < 64; x <<= 1) {
+      const f32x4 o = {__shfl_xor(st.o[0], x), __shfl_xor(st.o[1], x), __shfl_xor(st.o[2], x),
+                       __shfl_xor(st.o[3], x)};
+      st.add(__shfl_xor(st.m, x), __shfl_xor(st.l, x), o);
+    }
+    if (lane < kMergeCols) s_m[wave][lane] = st;
+    __syncthreads();  // c is uniform over the workgroup
+    if (threadIdx.x < kMergeCols) {
+      st = s_m[0][lane];
+#pragma unroll
+      for (int w = 1; w < kHeadsPerGroup; ++w) st.add(s_m[w][lane].m, s_m[w][lane].l, s_m[w][lane].o);
+      const float inv = st.l > 0.f ? 1.f / st.l : 0.f;
+      uint16_t* op = a.out + (int64_t)b * a.out_bstride + (int64_t)(h * a.group) * D +
+                     (int64_t)(it / D4) * D + col;
+      *reinterpret_cast<u32x2*>(op) =
+          u32x2{E::bits(st.o[0] * inv) | (E::bits(st.o[1] * inv) << 16),
+                E::bits(st.o[2] * inv) | (E::bits(st.o[3] * inv) << 16)};
+    }
+    __syncthreads();  // s_m is rewritten by the next run of columns
+  }
+}
+
+// The merge of up to kMergeAlone pieces by one workgroup, PB at a time.
 template <int DT, int D, int KI, int PB>
 __device__ __forceinline__ void merge_pieces(const AttnArgs& a, const int4 d) {
   using E = Elem<DT>;
@@ -1247,7 +1393,7 @@ __device__ __forceinline__ void merge_pieces(const AttnArgs& a, const int4 d) {
   const int h = grp * kHeadsPerGroup + blockIdx.y;
   if (h >= a.n_kv_heads) return;
   const int items = a.group * D4;
-  const int64_t slot0 = (int64_t)d.z + (int64_t)grp * a.batch + b;
+  const int64_t slot0 = (int64_t)(d.z & 0xffff) + (int64_t)grp * a.batch + b;
   const int hl0 = blockIdx.y * a.group;  // first query head of h within a slot
   // the partials as raw buffers: a piece's offset is a uniform (scalar)
   // stride, so the PB loads of a round share one vector offset per thread
@@ -1307,6 +1453,7 @@ __device__ __forceinline__ void merge_pieces(const AttnArgs& a, const int4 d) {
 
 template <int DT, int D, int KI, int PB>
 __global__ __launch_bounds__(64 * kHeadsPerGroup) void attention_combine_kernel(AttnArgs a) {
+  __shared__ MergeState s_m[kHeadsPerGroup][kMergeCols];
   const int4 d = a.desc[blockIdx.x];
   // an appending call: this thread's first new-row chunk, loaded ahead of the merge
   const int64_t total = a.knew ? new_row_chunks<D>(a) : 0;
@@ -1320,7 +1467,10 @@ __global__ __launch_bounds__(64 * kHeadsPerGroup) void attention_combine_kernel(
     len0 = a.seq_lens[r.b];
     if (a.plan_last) blk0 = a.plan_last[r.b];
   }
-  if (d.x >= 0) merge_pieces<DT, D, KI, PB>(a, d);  // uniform over the workgroup
+  if (d.x >= 0) {  // uniform over the workgroup
+    if (d.w > kMergeAlone) merge_pieces_shared<DT, D>(a, d, s_m);
+    else merge_pieces<DT, D, KI, PB>(a, d);
+  }
   if (c0 < total) {
     const NewRowChunk<D> r(a, c0);
     if (u32x4* p = r.dst(a, len0, blk0)) __builtin_nontemporal_store(v0, p);
@@ -1492,7 +1642,7 @@ int run_attention(void* out, int64_t out_batch_stride, const void* q, int64_t q_
   a.knew_span = a.vnew_span = 0;
   a.n_desc = n_wg;
   if (plan) {
-    if (desc_per_sequence(batch, n_groups, n_wg)) a.n_desc = batch * n_groups;
+    if (desc_per_sequence(batch, n_groups, n_wg)) a.n_desc = batch * n_groups + kPlanHelpers;
     const PlanLayout pl = plan_layout(batch, n_wg, nblk_max);
     if (plan_bytes < (uint64_t)pl.total) return AEGKV_ERR_INVALID_ARG;
     if (!aligned16(plan)) return AEGKV_ERR_MISALIGNED;
@@ -1736,8 +1886,7 @@ int aegkv_paged_decode_plan(const int32_t* block_tables, int32_t max_blocks,
   p.last = reinterpret_cast<int32_t*>(pb + pl.last);
   p.ids = reinterpret_cast<int32_t*>(pb + pl.ids);
   p.tags = reinterpret_cast<int32_t*>(pb + pl.tags);
-  const int64_t work = std::max<int64_t>(std::max<int64_t>((int64_t)n_wg * 64, (int64_t)batch * nblk_max),
-                                         (int64_t)batch * p.n_groups);
+  const int64_t work = std::max<int64_t>((int64_t)n_wg * 64, (int64_t)batch * nblk_max);
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(1024, (work + 255) / 256));
   hipLaunchKernelGGL(decode_plan_kernel, dim3(grid), dim3(64 * kHeadsPerGroup),
                      (size_t)(3 * batch + 2) * sizeof(int32_t), (hipStream_t)stream, p);

@@ -919,3 +919,29 @@ def test_flash_attn_with_kvcache_reuses_the_step_plan(device):
     torch.cuda.synchronize()
     assert torch.equal(storage.view(torch.int16), two.view(torch.int16))
     assert torch.equal(got.view(-1).view(torch.int16), ref_app.view(-1).view(torch.int16))
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(28, 4, 128), (16, 1, 64), (6, 2, 256), (4, 4, 64)])
+@pytest.mark.parametrize("lens,nwg", [
+    ([400], 24), ([400], 25), ([400], 33), ([4800], 300),    # pieces of about one block each
+    ([800, 3, 800, 20, 801], 130), ([800, 3, 800, 20, 801], 40)])
+def test_merge_shared_by_workgroups(device, Hq, Hkv, D, lens, nwg):
+    """Sequences cut into about 24 pieces (the most one workgroup merges
+    alone), just more, and more than one round of a shared merge; several long
+    sequences at once; the planned merge descriptors (per sequence, with
+    helpers) against the unplanned ones (per workgroup), bit for bit."""
+    rng = np.random.default_rng(nwg + D)
+    lens, tables, padded, q, kc, vc = _setup(rng, lens, Hq, Hkv, D, "bf16")
+    scale = 1.0 / math.sqrt(D)
+    dev = lambda x: to_device_bits(x, "bf16", device)  # noqa: E731
+    bt = torch.from_numpy(padded).to(device)
+    sl = torch.from_numpy(lens.astype(np.int32)).to(device)
+    ml = int(lens.max())
+    args = (dev(q), dev(kc), dev(vc))
+    one = A.paged_decode_attention(*args, bt, sl, scale, ml, n_workgroups=nwg)
+    plan = A.DecodePlan(bt, sl, ml, Hkv, nwg)
+    two = A.paged_decode_attention(*args, None, None, scale, ml, n_workgroups=nwg, plan=plan)
+    ref = ko.paged_decode_attention(ko.bits_to_float(q, "bf16"), ko.bits_to_float(kc, "bf16"),
+                                    ko.bits_to_float(vc, "bf16"), padded, lens, scale)
+    _check(to_bits(one), ref, "bf16")
+    assert np.array_equal(to_bits(one), to_bits(two))
