@@ -3,22 +3,23 @@
 // aegaeon/aegaeon/worker.py:410-418 and run inside the forward at :517-523).
 //
 // Work decomposition (persistent and balanced).  The batch's KV blocks are
-// laid end to end per group of kHeadsPerGroup kv heads, each sequence
+// laid end to end per group of 4, 2 or 1 kv heads (heads_per_group), each sequence
 // preceded by kSegmentCost charge positions for the cost of starting it:
 // position P = grp * W + cum[b] + kSegmentCost + j for block j of sequence b,
-// W = sum_b (ceil(len_b / 16) + kSegmentCost).  One workgroup per CU takes an
-// equal contiguous range of positions, so every CU does the same work in a
-// single round, and consecutive ranges land on different XCDs (workgroups are
-// dealt to the XCDs round-robin).  Each workgroup computes the prefix sums of
+// W = sum_b (ceil(len_b / 16) + kSegmentCost).  One workgroup of four waves per
+// CU takes an equal contiguous range of positions (with 2 or 1 heads per group,
+// 2 or 4 consecutive ranges), so every CU does the same work in a
+// single round, and consecutive workgroups land on different XCDs (workgroups
+// are dealt to the XCDs round-robin).  Each workgroup computes the prefix sums of
 // the batch itself (into LDS) and walks its range; a range may cut sequences,
 // whose pieces write fp32 partials (unnormalised O, running max in log2
-// units, sum).  A workgroup's range can continue at most one cut sequence (it
-// began before the range, so it holds the range's start), so each workgroup
+// units, sum).  A range can continue at most one cut sequence (it began before
+// the range, so it holds the range's start), so each range
 // leaves a 16-byte merge descriptor (or none; a plan instead holds one per
 // sequence, and some to help with long ones, when sequences are fewer than
-// workgroups), and a second kernel, one workgroup per descriptor and kv head,
+// ranges), and a second kernel, one workgroup per descriptor and kv head,
 // merges its pieces with log-sum-exp weights: up to kMergeAlone pieces by one
-// workgroup, more by several.  A sequence held by one workgroup is
+// workgroup, more by several.  A sequence held by one range is
 // normalised and written directly.  (Merging in the main kernel by the last
 // piece to arrive measured slower every way it was built: with device-scope
 // release fences, which write back the XCD's L2, 2x; with write-through
@@ -27,8 +28,8 @@
 // ordinary ones, and the last arrival's merge of a long sequence's pieces on
 // one CU ~10 us more, against ~3.6 us for this second launch.)
 //
-// Inside a workgroup, wave w handles kv head grp * 4 + w, and all
-// G = Hq / Hkv query heads of that kv head are processed together, so each K/V
+// Inside a workgroup of group size H, wave w handles kv head grp * H + w % H
+// over range w / H of the workgroup, and all G = Hq / Hkv query heads of that kv head are processed together, so each K/V
 // byte is read from HBM exactly once per decode step.  A wave streams the
 // blocks of its whole range through one register pipeline, across sequence
 // boundaries, and keeps the pieces it finishes in LDS until the stream ends
@@ -70,17 +71,18 @@ typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kBlockSize = 16;
-constexpr int kHeadsPerGroup = 4;   // waves (kv heads) per workgroup
+constexpr int kWaves = 4;           // waves per workgroup
 constexpr int kMaxBatch = 2048;     // sequences per launch (LDS prefix sums); larger
                                     // batches are launched in chunks
 constexpr int kMaxWorkgroups = 8192;  // bound of n_workgroups
+constexpr int kMaxRanges = kMaxWorkgroups * kWaves;
 constexpr int kMaxStage = 4;          // finished pieces a wave stages in LDS
 constexpr int kNewStage = 8;          // an appending call: sequences' new rows a wave stages in LDS
 // A raw buffer offset past every range this file builds (each below 2^31
 // bytes): the access returns zeros and reads no memory.
 constexpr uint32_t kPastRange = 0xFFFFFFF0u;
 constexpr int kStageBudget = 64 * 1024;  // dynamic LDS of a workgroup, scan arrays included
-constexpr int kScanPerThread = kMaxBatch / (64 * kHeadsPerGroup);
+constexpr int kScanPerThread = kMaxBatch / (64 * kWaves);
 // Cost of switching the block stream to a new sequence (its piece staged,
 // its query swapped in) in units of one block: the partition balances blocks
 // plus this charge per sequence, so a workgroup that holds several short
@@ -98,6 +100,17 @@ __device__ __forceinline__ int cost_units(int len) {
 // wave per SIMD.
 template <int D>
 constexpr int pipeline_depth() { return D >= 256 ? 2 : 3; }
+
+// kv heads of a workgroup's group, one per wave; the 4 / heads waves of each
+// head take ranges of their own.  The largest of 4, 2, 1 that divides the kv
+// heads, so that no wave idles (7 query heads over one kv head, 256 sequences
+// of 1000 tokens: 42.4 us per layer with one wave of four busy, 26.0
+// with four ranges); above 63 kv heads an idle wave or two per group of four
+// matter less than the range arithmetic's bound (positions_fit).
+inline int heads_per_group(int32_t n_kv_heads) {
+  if (n_kv_heads % 4 == 0 || n_kv_heads > 63) return 4;
+  return n_kv_heads % 2 == 0 ? 2 : 1;
+}
 constexpr float kRescaleSlack = 8.f;  // log2 headroom of the lazy softmax rescale
 
 template <int DT>
@@ -156,9 +169,12 @@ struct AttnArgs {
   int32_t n_kv_heads;
   int32_t head_dim;
   int32_t group;     // n_q_heads / n_kv_heads
-  int32_t hpg;       // query heads per workgroup: kHeadsPerGroup * group
-  int32_t n_groups;  // ceil(n_kv_heads / kHeadsPerGroup)
+  int32_t heads;     // kv heads per group (heads_per_group)
+  int32_t hpg;       // query heads per group: heads * group
+  int32_t n_groups;  // ceil(n_kv_heads / heads)
   int32_t n_wg;      // workgroups of the main kernel
+  int32_t splits;    // ranges per workgroup: kWaves / heads
+  int32_t n_ranges;  // n_wg * splits
   float scale_log2;  // softmax scale * log2(e)
   int32_t max_seq_len;  // host bound; longer device lengths are clamped to it
   uint16_t* out;
@@ -200,14 +216,14 @@ constexpr int kMergeAlone = 24;
 constexpr int kMaxHelpers = 64;  // workgroups (per kv head) that share one merge
 
 // Merge descriptor: sequence b of kv-head group grp, cut into np pieces held
-// by workgroups w0 .. w0 + np - 1; this descriptor's workgroup is number k of
-// the nh that merge it.  (np <= 2^15; b < 0: nothing to do.)
+// by ranges w0 .. w0 + np - 1; this descriptor's workgroup is number k of the
+// nh that merge it.  (np <= kMaxRanges = 2^15; b < 0: nothing to do.)
 __device__ __forceinline__ int4 merge_desc(int b, int grp, int w0, int np, int k, int nh) {
   return make_int4(b, grp, w0 | (k << 16) | (nh << 23), np);
 }
 __device__ __forceinline__ int4 no_merge() { return make_int4(-1, 0, 0, 0); }
-// The descriptor of workgroup w, whose range starts in sequence b of group
-// grp held by workgroups [w0, w1]: the last of them merges a short cut
+// The descriptor of range w, which starts in sequence b of group grp held by
+// ranges [w0, w1]: the last of them merges a short cut
 // sequence, the ones after the first share a long one's merge.
 __device__ __forceinline__ int4 continued_desc(int b, int grp, int64_t w0, int64_t w1, int64_t w) {
   const int np = (int)(w1 - w0 + 1);
@@ -219,22 +235,22 @@ __device__ __forceinline__ int4 continued_desc(int b, int grp, int64_t w0, int64
 
 // A plan indexes the merge descriptors by (kv-head group, sequence) when
 // those, with kPlanHelpers to share the merges of long sequences, are no more
-// than the workgroups, so that the combine grid is that much smaller (the
+// than the ranges, so that the combine grid is that much smaller (the
 // Qwen2.5-7B heads, 128 sequences: 160 descriptors against 256, 0.8 us per layer);
-// otherwise, and without a plan, by the workgroup that continues the sequence.
+// otherwise, and without a plan, by the range that continues the sequence.
 constexpr int kPlanHelpers = 32;
-// Long sequences of one launch: each takes more than kMergeAlone - 1 workgroups
-// beyond its first, and a workgroup continues at most one sequence.
-constexpr int kMaxLong = kMaxWorkgroups / kMergeAlone + 1;
-inline bool desc_per_sequence(int64_t batch, int64_t n_groups, int64_t n_wg) {
-  return batch * n_groups + kPlanHelpers <= n_wg;
+// Long sequences of one launch: each takes more than kMergeAlone - 1 ranges
+// beyond its first, and a range continues at most one sequence.
+constexpr int kMaxLong = kMaxRanges / kMergeAlone + 1;
+inline bool desc_per_sequence(int64_t batch, int64_t n_groups, int64_t n_ranges) {
+  return batch * n_groups + kPlanHelpers <= n_ranges;
 }
 
-// Decode plan, in one device buffer: per main-kernel workgroup a record of 8
-// int32 (first kv-head group or -1 for an idle workgroup, last group, first
+// Decode plan, in one device buffer: per range a record of 8
+// int32 (first kv-head group or -1 for an idle range, last group, first
 // item and its sequence, end item in the last group, the batch's first
 // non-empty sequence), the merge descriptors, the block ids and new-row tags
-// of the first 64 items of each workgroup's range, the id of the block that
+// of the first 64 items of each range, the id of the block that
 // holds each sequence's position seq_lens[b] - 1 (-1 when empty or past its
 // table), the block ids of all items in item order (item i = block
 // i - bcum[b] of the sequence b holding it), and their new-row tags (b * 16 +
@@ -245,33 +261,33 @@ inline bool desc_per_sequence(int64_t batch, int64_t n_groups, int64_t n_wg) {
 struct PlanLayout {
   int64_t wg, desc, first, last, ids, tags, total;
 };
-inline PlanLayout plan_layout(int64_t batch, int64_t n_wg, int64_t nblk_max) {
+inline PlanLayout plan_layout(int64_t batch, int64_t n_ranges, int64_t nblk_max) {
   auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
   PlanLayout l;
   l.wg = 0;
-  l.desc = up(n_wg * 32);
-  l.first = l.desc + up(n_wg * 16);
-  l.last = l.first + up(n_wg * 128 * 4);
+  l.desc = up(n_ranges * 32);
+  l.first = l.desc + up(n_ranges * 16);
+  l.last = l.first + up(n_ranges * 128 * 4);
   l.ids = l.last + up(batch * 4);
   l.tags = l.ids + up(batch * nblk_max * 4);
   l.total = l.tags + up(batch * nblk_max * 4);
   return l;
 }
-constexpr int kPlanRecord = 8;  // int32 per workgroup record
+constexpr int kPlanRecord = 8;  // int32 per range record
 
-// Workspace layout of one launch: the workgroups' descriptors, then the
-// partials of n_wg + n_groups * batch slots (a workgroup writes at most one
-// slot per sequence piece it holds; slot = workgroup + grp * batch + b is
+// Workspace layout of one launch: the ranges' descriptors, then the
+// partials of n_ranges + n_groups * batch slots (a range writes at most one
+// slot per sequence piece it holds; slot = range + grp * batch + b is
 // unique).  Every byte the combine reads is written by the same launch.
 struct WorkspaceLayout {
   int64_t desc_bytes, ml_bytes, o_bytes, total;
 };
 inline WorkspaceLayout workspace_layout(int64_t batch, int64_t hpg, int64_t head_dim,
-                                        int64_t n_wg, int64_t n_groups) {
+                                        int64_t n_ranges, int64_t n_groups) {
   auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
-  const int64_t slots = n_wg + n_groups * batch;
+  const int64_t slots = n_ranges + n_groups * batch;
   WorkspaceLayout w;
-  w.desc_bytes = up(n_wg * 16);
+  w.desc_bytes = up(n_ranges * 16);
   w.ml_bytes = up(slots * hpg * 8);
   w.o_bytes = up(slots * hpg * head_dim * 4);
   w.total = w.desc_bytes + w.ml_bytes + w.o_bytes;
@@ -530,9 +546,9 @@ __device__ __forceinline__ void get_record(const uint8_t* rec, f32x4* acc, float
   lt = ml.y;
 }
 
-// One wave's share of a workgroup's range within kv-head group `grp`: block
+// One wave's share of range `range` within kv-head group `grp`: block
 // items [i0, i1) of the group, item i being block i - bcum[b] of the sequence
-// b with bcum[b] <= i < bcum[b + 1], for kv head grp * 4 + wave.
+// b with bcum[b] <= i < bcum[b + 1], for head `hl` of the group's a.heads.
 //
 // The items are streamed through one rolling register pipeline of NBUF
 // blocks whatever the sequence boundaries: buffer k holds item i0 + it + k;
@@ -556,21 +572,21 @@ __device__ __forceinline__ void get_record(const uint8_t* rec, f32x4* acc, float
 template <int DT, int D, int NBUF, bool PLANNED, bool FUSED>
 __device__ __forceinline__ void attend_items(const AttnArgs& a, const int32_t* s_bcum,
                                              const int32_t* s_len, uint8_t* stage, int4* meta,
-                                             int grp, int b0, int i0, int i1, bool have_first,
-                                             int id_first, int tag_first,
+                                             int range, int grp, int hl, int b0, int i0, int i1,
+                                             bool have_first, int id_first, int tag_first,
                                              const uint32_t* s_over = nullptr,
                                              uint8_t* nstage = nullptr, int32_t* nseq = nullptr) {
   constexpr int KS = D / 32;
   constexpr int DPL = D / 16;
   constexpr bool kNewInLds = FUSED && D <= 128;  // an appending call's rows staged in LDS
   constexpr bool kTags = FUSED && !kNewInLds;     // per-item new-row tags (D = 256)
-  const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
-  const int h = grp * kHeadsPerGroup + wave;
+  const int lane = threadIdx.x & 63;
+  const int h = grp * a.heads + hl;
   if (h >= a.n_kv_heads) return;  // wave past the last kv head (uniform)
   const int j = lane & 15, g = lane >> 4;
   const bool head_ok = j < a.group;
   const int hq = h * a.group + j;
-  const int hl0 = wave * a.group;
+  const int hl0 = hl * a.group;
   const int64_t row = (int64_t)a.n_kv_heads * D;
   const uint32_t row_b = (uint32_t)(row * 2);
   const uint32_t blk_b = kBlockSize * row_b;  // a block's K (or V) rows
@@ -780,7 +796,7 @@ __device__ __forceinline__ void attend_items(const AttnArgs& a, const int32_t* s
     if (++ic == cend) {  // the piece of sequence bc in this range ends (uniform)
       float lt = lsum + __shfl_xor(lsum, 16);
       lt += __shfl_xor(lt, 32);
-      const int pslot = (int)blockIdx.x + grp * a.batch + bc;
+      const int pslot = range + grp * a.batch + bc;
       if (stages_pieces<D>() && a.stage_slots > 0) {
         if (nstaged == a.stage_slots) flush();
         if (head_ok) put_record<D>(my_rec + nstaged * slot_bytes, acc, m, lt);
@@ -876,21 +892,21 @@ __device__ __forceinline__ void attend_items(const AttnArgs& a, const int32_t* s
 // max_seq_len) into LDS: s_cum[batch + 1] (cost units), s_bcum[batch + 1]
 // (blocks), s_len[batch]; with s_over, bit b set when sequence b's length
 // exceeds max_seq_len (its last token, an appending call's new row, then lies
-// past the attended range).  Every thread of the 64 * kHeadsPerGroup takes
+// past the attended range).  Every thread of the 64 * kWaves takes
 // part.
 __device__ __forceinline__ void scan_batch(const int32_t* seq_lens, int batch, int max_seq_len,
                                            int32_t* s_cum, int32_t* s_bcum, int32_t* s_len,
-                                           int32_t (*s_wave_tot)[kHeadsPerGroup],
+                                           int32_t (*s_wave_tot)[kWaves],
                                            uint32_t* s_over = nullptr) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
   if (s_over)
-    for (int w = tid; w < kMaxBatch / 32; w += 64 * kHeadsPerGroup) s_over[w] = 0u;
+    for (int w = tid; w < kMaxBatch / 32; w += 64 * kWaves) s_over[w] = 0u;
   // Prefix sums of the batch's positions and blocks: thread t owns sequences
   // [t * per, t * per + per); a wave scan plus the wave totals give each
   // thread its exclusive offsets.
   {
-    const int per = (batch + 64 * kHeadsPerGroup - 1) / (64 * kHeadsPerGroup);
+    const int per = (batch + 64 * kWaves - 1) / (64 * kWaves);
     const int b0 = tid * per;
     int lens[kScanPerThread];
     int cnt = 0, bcnt = 0;
@@ -936,7 +952,7 @@ __device__ __forceinline__ void scan_batch(const int32_t* seq_lens, int batch, i
         bexcl += (lens[k] + kBlockSize - 1) / kBlockSize;
       }
     }
-    if (tid == 64 * kHeadsPerGroup - 1) {
+    if (tid == 64 * kWaves - 1) {
       s_cum[batch] = base + x;
       s_bcum[batch] = bbase + y;
     }
@@ -963,31 +979,32 @@ __device__ __forceinline__ int64_t owner_of(int64_t P, int64_t total, int64_t n_
 }
 
 template <int DT, int D, int NBUF, bool PLANNED, bool FUSED>
-__global__ __launch_bounds__(64 * kHeadsPerGroup, D >= 256 ? 1 : 2) void
+__global__ __launch_bounds__(64 * kWaves, D >= 256 ? 1 : 2) void
 paged_decode_attention_kernel(AttnArgs a) {
   // cum[batch + 1] (positions), len[batch], bcum[batch + 1] (blocks)
   extern __shared__ int32_t s_mem[];
-  __shared__ int32_t s_wave_tot[2][kHeadsPerGroup];
-  __shared__ int32_t s_find[2];
-  __shared__ int4 s_meta[kHeadsPerGroup][kMaxStage];
+  __shared__ int32_t s_wave_tot[2][kWaves];
+  __shared__ int4 s_meta[kWaves][kMaxStage];
   __shared__ uint32_t s_over[FUSED ? kMaxBatch / 32 : 1];
-  __shared__ int32_t s_newseq[kHeadsPerGroup][FUSED ? kNewStage : 1];
+  __shared__ int32_t s_newseq[kWaves][FUSED ? kNewStage : 1];
   int32_t* s_cum = s_mem;
   int32_t* s_len = s_mem + a.batch + 1;
   int32_t* s_bcum = s_len + a.batch;
   const int tid = threadIdx.x;
-  const int lane = tid & 63, wave = tid >> 6;
+  const int lane = tid & 63, wave = uni(tid >> 6);
+  // the wave's range and its kv head within a group
+  const int range = (int)blockIdx.x * a.splits + wave / a.heads, hl = wave % a.heads;
 
-  // A planned workgroup's record and the block ids of its first 64 items,
+  // A planned range's record and the block ids of its first 64 items,
   // loaded before the scan so that they arrive while it runs.
   int rec[kPlanRecord] = {};
   int id_first = 0, tag_first = -1;
   if constexpr (PLANNED) {
 #pragma unroll
-    for (int k = 0; k < kPlanRecord; ++k) rec[k] = a.plan_wg[(int64_t)blockIdx.x * kPlanRecord + k];
-    id_first = a.plan_first[(int64_t)blockIdx.x * 128 + lane];
+    for (int k = 0; k < kPlanRecord; ++k) rec[k] = a.plan_wg[(int64_t)range * kPlanRecord + k];
+    id_first = a.plan_first[(int64_t)range * 128 + lane];
     if constexpr (FUSED && D > 128)  // per-item tags: the lane-select path only
-      tag_first = a.plan_first[(int64_t)blockIdx.x * 128 + 64 + lane];
+      tag_first = a.plan_first[(int64_t)range * 128 + 64 + lane];
   }
   scan_batch(a.seq_lens, a.batch, a.max_seq_len, s_cum, s_bcum, s_len, s_wave_tot,
              FUSED ? s_over : nullptr);
@@ -995,7 +1012,7 @@ paged_decode_attention_kernel(AttnArgs a) {
   for (int b = blockIdx.x; b < a.batch; b += gridDim.x) {
     if (s_cum[b + 1] != s_cum[b]) continue;  // uniform over the workgroup
     uint16_t* op = a.out + (int64_t)b * a.out_bstride;
-    for (int e = tid * 8; e < a.n_q_heads * a.head_dim; e += 8 * 64 * kHeadsPerGroup)
+    for (int e = tid * 8; e < a.n_q_heads * a.head_dim; e += 8 * 64 * kWaves)
       *reinterpret_cast<u32x4*>(op + e) = u32x4{0u, 0u, 0u, 0u};
   }
 
@@ -1003,7 +1020,7 @@ paged_decode_attention_kernel(AttnArgs a) {
                    wave * a.stage_slots * a.group * 4 * stage_record_bytes<D>();
   uint8_t* nstage = reinterpret_cast<uint8_t*>(s_mem) + a.newrow_off + wave * kNewStage * 4 * D;
   if constexpr (PLANNED) {
-    if (uni(rec[0]) < 0) return;  // idle workgroup
+    if (uni(rec[0]) < 0) return;  // idle range
     const int items = s_bcum[a.batch];
     for (int grp = uni(rec[0]); grp <= uni(rec[1]); ++grp) {
       const bool first_pass = grp == uni(rec[0]);
@@ -1011,8 +1028,8 @@ paged_decode_attention_kernel(AttnArgs a) {
       const int b0 = first_pass ? uni(rec[3]) : uni(rec[5]);
       const int i1 = grp == uni(rec[1]) ? uni(rec[4]) : items;
       if (i1 > i0)
-        attend_items<DT, D, NBUF, true, FUSED>(a, s_bcum, s_len, stage, s_meta[wave], grp, b0,
-                                               i0, i1, first_pass, id_first,
+        attend_items<DT, D, NBUF, true, FUSED>(a, s_bcum, s_len, stage, s_meta[wave], range, grp,
+                                               hl, b0, i0, i1, first_pass, id_first,
                                                first_pass ? tag_first : -1, s_over, nstage,
                                                s_newseq[wave]);
     }
@@ -1020,55 +1037,54 @@ paged_decode_attention_kernel(AttnArgs a) {
   }
   const int64_t W = s_cum[a.batch];
   const int64_t total = W * a.n_groups;
-  // With fewer positions than workgroups only the first `total` take part, so
+  // With fewer positions than ranges only the first `total` take part, so
   // that every range is non-empty.
-  const int64_t n_act = min((int64_t)a.n_wg, total);
-  if ((int64_t)blockIdx.x >= n_act) {
-    if (tid == 0) a.desc[blockIdx.x] = no_merge();
+  const int64_t n_act = min((int64_t)a.n_ranges, total);
+  if (range >= n_act) {
+    if (hl == 0 && lane == 0) a.desc[range] = no_merge();
     return;
   }
-  int64_t P = div_floor((int64_t)blockIdx.x * total, n_act);
-  const int64_t p_end = div_floor((int64_t)(blockIdx.x + 1) * total, n_act);
-  // Every value below is uniform over the workgroup.  A sequence occupies
+  int64_t P = div_floor((int64_t)range * total, n_act);
+  const int64_t p_end = div_floor((int64_t)(range + 1) * total, n_act);
+  // Every value below is uniform over the wave.  A sequence occupies
   // positions [s_cum[b], s_cum[b + 1]) of its group: kSegmentCost charge
   // positions, then one per block.
+  auto items_before = [&](int b, int p) -> int {  // block items before position p of sequence b
+    const int nblk = s_bcum[b + 1] - s_bcum[b];
+    return s_bcum[b] + min(max(p - s_cum[b] - kSegmentCost, 0), nblk);
+  };
+  auto seq_of = [&](int p) -> int {  // the sequence holding position p < W, by every lane's test
+    int b = 0;
+    for (int base = 0; base < a.batch; base += 64) {
+      const int c = base + lane;
+      const uint64_t hit =
+          __builtin_amdgcn_ballot_w64(c < a.batch && s_cum[c] <= p && p < s_cum[c + 1]);
+      if (hit) b = base + __builtin_ctzll(hit);
+    }
+    return uni(b);
+  };
   bool first_pass = true;
   while (P < p_end) {  // one pass per kv-head group the range touches
     const int grp = (int)div_floor(P, W);
     const int64_t pbase = (int64_t)grp * W;
     const int64_t q_end = min(p_end, pbase + W);
     const int p0 = (int)(P - pbase), p1 = (int)(q_end - pbase);
-    // the sequences holding positions p0 and p1 (p1 < W), every thread
-    // testing its own sequences at once
-    for (int b = tid; b < a.batch; b += 64 * kHeadsPerGroup) {
-      const int lo = s_cum[b], hi = s_cum[b + 1];
-      if (lo <= p0 && p0 < hi) s_find[0] = b;
-      if (lo <= p1 && p1 < hi) s_find[1] = b;
-    }
-    __syncthreads();
-    // block items before position p of sequence b
-    auto items_before = [&](int b, int p) -> int {
-      const int nblk = s_bcum[b + 1] - s_bcum[b];
-      return s_bcum[b] + min(max(p - s_cum[b] - kSegmentCost, 0), nblk);
-    };
-    const int b0 = s_find[0];
-    const int i0 = items_before(b0, p0);
-    const int i1 = p1 == (int)W ? s_bcum[a.batch] : items_before(s_find[1], p1);
+    const int b0 = seq_of(p0);
+    const int i0 = uni(items_before(b0, p0));
+    const int i1 = uni(p1 == (int)W ? s_bcum[a.batch] : items_before(seq_of(p1), p1));
     if (first_pass) {
       // The range's first piece is the only one that can continue a cut
       // sequence: describe it for the merge when it does.
       const int64_t w0 = owner_of(pbase + s_cum[b0] + kSegmentCost, total, n_act);
       const int64_t w1 = owner_of(pbase + s_cum[b0 + 1] - 1, total, n_act);
-      if (tid == 0)
-        a.desc[blockIdx.x] = continued_desc(b0, grp, w0, w1, (int64_t)blockIdx.x);
+      if (hl == 0 && lane == 0) a.desc[range] = continued_desc(b0, grp, w0, w1, range);
       first_pass = false;
     }
     if (i1 > i0)
-      attend_items<DT, D, NBUF, false, FUSED>(a, s_bcum, s_len, stage, s_meta[wave], grp, b0,
-                                              i0, i1, false, 0, -1, s_over, nstage,
+      attend_items<DT, D, NBUF, false, FUSED>(a, s_bcum, s_len, stage, s_meta[wave], range, grp,
+                                              hl, b0, i0, i1, false, 0, -1, s_over, nstage,
                                               s_newseq[wave]);
     P = q_end;
-    __syncthreads();  // s_find is rewritten by the next pass
   }
 }
 
@@ -1079,8 +1095,8 @@ struct PlanArgs {
   int32_t batch;
   int32_t max_seq_len;
   int32_t n_groups;
-  int32_t n_wg;
-  int32_t desc_per_seq;  // descriptors indexed by grp * batch + b (else by workgroup)
+  int32_t n_ranges;
+  int32_t desc_per_seq;  // descriptors indexed by grp * batch + b (else by range)
   int32_t* wg;
   int4* desc;
   int32_t* first;
@@ -1091,11 +1107,11 @@ struct PlanArgs {
 
 // Builds a decode plan (see PlanLayout) with the partition the attention
 // kernel computes for itself: every workgroup scans the lengths, then the
-// grid shares the per-workgroup records, the first-64 id lists and the
+// grid shares the per-range records, the first-64 id lists and the
 // item-order ids.
-__global__ __launch_bounds__(64 * kHeadsPerGroup) void decode_plan_kernel(PlanArgs p) {
+__global__ __launch_bounds__(64 * kWaves) void decode_plan_kernel(PlanArgs p) {
   extern __shared__ int32_t s_mem[];
-  __shared__ int32_t s_wave_tot[2][kHeadsPerGroup];
+  __shared__ int32_t s_wave_tot[2][kWaves];
   __shared__ uint32_t s_over[kMaxBatch / 32];
   int32_t* s_cum = s_mem;
   int32_t* s_len = s_mem + p.batch + 1;
@@ -1104,14 +1120,14 @@ __global__ __launch_bounds__(64 * kHeadsPerGroup) void decode_plan_kernel(PlanAr
   const int64_t W = s_cum[p.batch];
   const int items = s_bcum[p.batch];
   const int64_t total = W * p.n_groups;
-  const int64_t n_act = min((int64_t)p.n_wg, total);
+  const int64_t n_act = min((int64_t)p.n_ranges, total);
   const int gtid = blockIdx.x * blockDim.x + threadIdx.x;
   const int gsz = gridDim.x * blockDim.x;
   auto items_before = [&](int b, int pos) -> int {
     const int nblk = s_bcum[b + 1] - s_bcum[b];
     return s_bcum[b] + min(max(pos - s_cum[b] - kSegmentCost, 0), nblk);
   };
-  // workgroup w's range: first and last kv-head group, first item and its
+  // range w: first and last kv-head group, first item and its
   // sequence, end item in the last group and in the first
   struct Range {
     int gf, gl, i0, b0, i1l, i1f;
@@ -1130,7 +1146,7 @@ __global__ __launch_bounds__(64 * kHeadsPerGroup) void decode_plan_kernel(PlanAr
     r.i1f = r.gf == r.gl ? r.i1l : items;
     return r;
   };
-  for (int w = gtid; w < p.n_wg; w += gsz) {
+  for (int w = gtid; w < p.n_ranges; w += gsz) {
     int32_t* rec = p.wg + (int64_t)w * kPlanRecord;
     if (w >= n_act) {
       rec[0] = -1;
@@ -1202,7 +1218,7 @@ __global__ __launch_bounds__(64 * kHeadsPerGroup) void decode_plan_kernel(PlanAr
     return i == s_bcum[b + 1] - 1 && !((s_over[b >> 5] >> (b & 31)) & 1u)
                ? b * kBlockSize + ((s_len[b] - 1) & (kBlockSize - 1)) : -1;
   };
-  for (int64_t e = gtid; e < (int64_t)p.n_wg * 64; e += gsz) {
+  for (int64_t e = gtid; e < (int64_t)p.n_ranges * 64; e += gsz) {
     const int w = (int)(e >> 6);
     if (w >= n_act) continue;
     const Range r = range_of(w);
@@ -1226,7 +1242,7 @@ __global__ __launch_bounds__(64 * kHeadsPerGroup) void decode_plan_kernel(PlanAr
 }
 
 // Merge the pieces of the cut sequence that descriptor blockIdx.x names
-// (none: nothing to do), for kv head grp * 4 + blockIdx.y:
+// (none: nothing to do), for kv head grp * a.heads + blockIdx.y:
 //   out = sum_s w_s o_s / sum_s w_s l_s,  w_s = 2^(m_s - max m).
 // The kv head's G query heads x D/4 float4 columns are "items", one per
 // thread (KI per thread past 256 items); a thread loads the (m, l) and o of
@@ -1297,7 +1313,7 @@ __device__ __forceinline__ int64_t new_row_chunks(const AttnArgs& a) {
 // piece each and meet through shuffles and LDS.  The sums' order does not
 // depend on nh, so every launch form gives the same bits.
 constexpr int kMergeCols = 8;
-constexpr int kMergeSlices = 64 * kHeadsPerGroup / kMergeCols;
+constexpr int kMergeSlices = 64 * kWaves / kMergeCols;
 constexpr int kMergeAhead = 8;  // pieces a thread loads at once
 struct MergeState {
   float m, l;
@@ -1318,7 +1334,7 @@ __device__ __forceinline__ void merge_pieces_shared(const AttnArgs& a, const int
   using E = Elem<DT>;
   constexpr int D4 = D / 4;
   const int b = d.x, grp = d.y, npieces = d.w;
-  const int h = grp * kHeadsPerGroup + blockIdx.y;
+  const int h = grp * a.heads + blockIdx.y;
   if (h >= a.n_kv_heads) return;
   const int w0 = d.z & 0xffff, nh = (int)((uint32_t)d.z >> 23);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -1371,7 +1387,7 @@ __device__ __forceinline__ void merge_pieces_shared(const AttnArgs& a, const int
     if (threadIdx.x < kMergeCols) {
       st = s_m[0][lane];
 #pragma unroll
-      for (int w = 1; w < kHeadsPerGroup; ++w) st.add(s_m[w][lane].m, s_m[w][lane].l, s_m[w][lane].o);
+      for (int w = 1; w < kWaves; ++w) st.add(s_m[w][lane].m, s_m[w][lane].l, s_m[w][lane].o);
       const float inv = st.l > 0.f ? 1.f / st.l : 0.f;
       uint16_t* op = a.out + (int64_t)b * a.out_bstride + (int64_t)(h * a.group) * D +
                      (int64_t)(it / D4) * D + col;
@@ -1388,9 +1404,9 @@ template <int DT, int D, int KI, int PB>
 __device__ __forceinline__ void merge_pieces(const AttnArgs& a, const int4 d) {
   using E = Elem<DT>;
   constexpr int D4 = D / 4;  // float4 per query head
-  constexpr int NT = 64 * kHeadsPerGroup;
+  constexpr int NT = 64 * kWaves;
   const int b = d.x, grp = d.y, npieces = d.w;
-  const int h = grp * kHeadsPerGroup + blockIdx.y;
+  const int h = grp * a.heads + blockIdx.y;
   if (h >= a.n_kv_heads) return;
   const int items = a.group * D4;
   const int64_t slot0 = (int64_t)(d.z & 0xffff) + (int64_t)grp * a.batch + b;
@@ -1452,8 +1468,8 @@ __device__ __forceinline__ void merge_pieces(const AttnArgs& a, const int4 d) {
 }
 
 template <int DT, int D, int KI, int PB>
-__global__ __launch_bounds__(64 * kHeadsPerGroup) void attention_combine_kernel(AttnArgs a) {
-  __shared__ MergeState s_m[kHeadsPerGroup][kMergeCols];
+__global__ __launch_bounds__(64 * kWaves) void attention_combine_kernel(AttnArgs a) {
+  __shared__ MergeState s_m[kWaves][kMergeCols];
   const int4 d = a.desc[blockIdx.x];
   // an appending call: this thread's first new-row chunk, loaded ahead of the merge
   const int64_t total = a.knew ? new_row_chunks<D>(a) : 0;
@@ -1488,9 +1504,9 @@ __global__ __launch_bounds__(64 * kHeadsPerGroup) void attention_combine_kernel(
 // a.stage_off and a.newrow_off.
 size_t lds_bytes(AttnArgs& a, int max_lds) {
   const int64_t scan = ((int64_t)(3 * a.batch + 2) * (int64_t)sizeof(int32_t) + 15) / 16 * 16;
-  const int64_t per_slot = (int64_t)kHeadsPerGroup * a.group * 4 * (a.head_dim + 16);
+  const int64_t per_slot = (int64_t)kWaves * a.group * 4 * (a.head_dim + 16);
   const int64_t newrows =
-      a.knew && a.head_dim <= 128 ? (int64_t)kHeadsPerGroup * kNewStage * 4 * a.head_dim : 0;
+      a.knew && a.head_dim <= 128 ? (int64_t)kWaves * kNewStage * 4 * a.head_dim : 0;
   const int64_t budget = std::min<int64_t>(kStageBudget, max_lds - newrows) - scan;
   a.stage_off = (int32_t)scan;
   a.stage_slots = a.head_dim > 128 ? 0
@@ -1516,17 +1532,17 @@ int workgroups_for(int32_t requested, int* n_wg) {
 
 // The kernel's position arithmetic: a group's positions W (bounded by
 // chunk * (blocks + kSegmentCost)) must fit int32, and the products of the
-// range arithmetic (total * n_wg, total = W * n_groups) must stay below 2^52
-// for div_floor.
-bool positions_fit(int64_t chunk, int64_t nblk_max, int64_t n_groups, int64_t n_wg) {
+// range arithmetic (total * n_ranges, total = W * n_groups) must stay below
+// 2^52 for div_floor.
+bool positions_fit(int64_t chunk, int64_t nblk_max, int64_t n_groups, int64_t n_ranges) {
   const int64_t w_max = chunk * (nblk_max + kSegmentCost);
-  return w_max < (1ll << 31) && w_max * n_groups * n_wg < (1ll << 52);
+  return w_max < (1ll << 31) && w_max * n_groups * n_ranges < (1ll << 52);
 }
 
 template <int DT, int D, int KI, int PB>
 int launch_combine(const AttnArgs& a, hipStream_t stream) {
   hipLaunchKernelGGL((attention_combine_kernel<DT, D, KI, PB>),
-                     dim3(a.n_desc, kHeadsPerGroup), dim3(64 * kHeadsPerGroup), 0,
+                     dim3(a.n_desc, a.heads), dim3(64 * kWaves), 0,
                      stream, a);
   AEGKV_HIP_TRY(hipGetLastError());
   return AEGKV_OK;
@@ -1535,7 +1551,7 @@ int launch_combine(const AttnArgs& a, hipStream_t stream) {
 template <int DT, int D, bool PLANNED, bool FUSED>
 void launch_main(const AttnArgs& a, size_t lds, hipStream_t stream) {
   hipLaunchKernelGGL((paged_decode_attention_kernel<DT, D, pipeline_depth<D>(), PLANNED, FUSED>),
-                     dim3(a.n_wg), dim3(64 * kHeadsPerGroup), lds, stream, a);
+                     dim3(a.n_wg), dim3(64 * kWaves), lds, stream, a);
 }
 
 template <int DT, int D>
@@ -1549,8 +1565,8 @@ int launch_attention(const AttnArgs& a, size_t lds, hipStream_t stream) {
   }
   AEGKV_HIP_TRY(hipGetLastError());
   const int items = a.group * (D / 4);  // <= 16 * D / 4
-  if (items <= 64 * kHeadsPerGroup) return launch_combine<DT, D, 1, 12>(a, stream);
-  if (items <= 2 * 64 * kHeadsPerGroup) return launch_combine<DT, D, 2, 12>(a, stream);
+  if (items <= 64 * kWaves) return launch_combine<DT, D, 1, 12>(a, stream);
+  if (items <= 2 * 64 * kWaves) return launch_combine<DT, D, 2, 12>(a, stream);
   return launch_combine<DT, D, 4, 12>(a, stream);
 }
 
@@ -1576,7 +1592,7 @@ int run_attention(void* out, int64_t out_batch_stride, const void* q, int64_t q_
                   int32_t max_seq_len, int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim,
                   int32_t block_size, float scale, int32_t dtype, int32_t n_workgroups,
                   void* workspace, uint64_t workspace_bytes, aegkv_stream_t stream,
-                  const NewRows& nr = NewRows()) {
+                  const NewRows& nr = NewRows(), int32_t heads = 0) {
   if (batch < 0 || max_seq_len < 0 || n_q_heads <= 0 || n_kv_heads <= 0 || max_blocks < 0 ||
       n_blocks < 0 || n_workgroups < 0)
     return AEGKV_ERR_INVALID_ARG;
@@ -1609,10 +1625,12 @@ int run_attention(void* out, int64_t out_batch_stride, const void* q, int64_t q_
   int rc = workgroups_for(n_workgroups, &n_wg);
   if (rc) return rc;
   const int32_t group = n_q_heads / n_kv_heads;
-  const int32_t n_groups = (n_kv_heads + kHeadsPerGroup - 1) / kHeadsPerGroup;
-  if (!positions_fit(chunk, nblk_max, n_groups, n_wg)) return AEGKV_ERR_UNSUPPORTED;
+  if (heads == 0) heads = heads_per_group(n_kv_heads);  // the caller's choice needs no plan
+  const int32_t n_groups = (n_kv_heads + heads - 1) / heads;
+  const int32_t n_ranges = n_wg * (kWaves / heads);
+  if (!positions_fit(chunk, nblk_max, n_groups, n_ranges)) return AEGKV_ERR_UNSUPPORTED;
   const WorkspaceLayout lay =
-      workspace_layout(chunk, kHeadsPerGroup * group, head_dim, n_wg, n_groups);
+      workspace_layout(chunk, heads * group, head_dim, n_ranges, n_groups);
   if (!workspace || workspace_bytes < (uint64_t)lay.total) return AEGKV_ERR_WORKSPACE;
   if (!aligned16(workspace)) return AEGKV_ERR_MISALIGNED;
   uint8_t* ws = static_cast<uint8_t*>(workspace);
@@ -1626,9 +1644,12 @@ int run_attention(void* out, int64_t out_batch_stride, const void* q, int64_t q_
   a.n_kv_heads = n_kv_heads;
   a.head_dim = head_dim;
   a.group = group;
-  a.hpg = kHeadsPerGroup * group;
+  a.heads = heads;
+  a.hpg = heads * group;
   a.n_groups = n_groups;
   a.n_wg = n_wg;
+  a.splits = kWaves / heads;
+  a.n_ranges = n_ranges;
   a.scale_log2 = scale * 1.4426950408889634f;
   a.max_seq_len = max_seq_len;
   a.q_bstride = q_batch_stride;
@@ -1640,10 +1661,10 @@ int run_attention(void* out, int64_t out_batch_stride, const void* q, int64_t q_
   a.knew_bstride = nr.key_bstride;
   a.vnew_bstride = nr.value_bstride;
   a.knew_span = a.vnew_span = 0;
-  a.n_desc = n_wg;
+  a.n_desc = n_ranges;
   if (plan) {
-    if (desc_per_sequence(batch, n_groups, n_wg)) a.n_desc = batch * n_groups + kPlanHelpers;
-    const PlanLayout pl = plan_layout(batch, n_wg, nblk_max);
+    if (desc_per_sequence(batch, n_groups, n_ranges)) a.n_desc = batch * n_groups + kPlanHelpers;
+    const PlanLayout pl = plan_layout(batch, n_ranges, nblk_max);
     if (plan_bytes < (uint64_t)pl.total) return AEGKV_ERR_INVALID_ARG;
     if (!aligned16(plan)) return AEGKV_ERR_MISALIGNED;
     const uint8_t* pb = static_cast<const uint8_t*>(plan);
@@ -1696,6 +1717,31 @@ int run_attention(void* out, int64_t out_batch_stride, const void* q, int64_t q_
   }
   return AEGKV_OK;
 }
+
+// Workspace bytes of one call with `heads` kv heads per group, or a status.
+int64_t workspace_size(int32_t batch, int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim,
+                       int32_t max_seq_len, int32_t dtype, int32_t n_workgroups, int32_t heads) {
+  if (batch < 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_q_heads % n_kv_heads ||
+      n_workgroups < 0 || max_seq_len < 0)
+    return AEGKV_ERR_INVALID_ARG;
+  if (n_workgroups > kMaxWorkgroups) return AEGKV_ERR_UNSUPPORTED;
+  if ((head_dim != 64 && head_dim != 128 && head_dim != 256) ||
+      (dtype != AEGKV_DTYPE_BF16 && dtype != AEGKV_DTYPE_FP16) || n_q_heads / n_kv_heads > 16)
+    return AEGKV_ERR_UNSUPPORTED;
+  if (batch == 0) return 0;
+  const int32_t chunk = std::min(batch, kMaxBatch);
+  int n_wg = 0;
+  const int rc = workgroups_for(n_workgroups, &n_wg);
+  if (rc) return rc > 0 ? AEGKV_ERR_RUNTIME : rc;
+  const int32_t group = n_q_heads / n_kv_heads;
+  const int32_t n_groups = (n_kv_heads + heads - 1) / heads;
+  const int32_t n_ranges = n_wg * (kWaves / heads);
+  if (!positions_fit(chunk, ((int64_t)max_seq_len + kBlockSize - 1) / kBlockSize, n_groups,
+                     n_ranges))
+    return AEGKV_ERR_UNSUPPORTED;
+  return workspace_layout(chunk, heads * group, head_dim, n_ranges, n_groups).total;
+}
+
 // Workspace of aegkv_paged_decode_attention_noalloc, held by the library in
 // device memory it never allocates: the merge descriptors and fp32 partials of
 // one call (the same layout the caller's workspace holds).  Every GPU the
@@ -1742,8 +1788,16 @@ int aegkv_paged_decode_attention_noalloc(void* out, int64_t out_batch_stride, co
                                          int32_t n_kv_heads, int32_t head_dim,
                                          int32_t block_size, float scale, int32_t dtype,
                                          int32_t n_workgroups, aegkv_stream_t stream) {
-  const int64_t need = aegkv_paged_decode_attention_workspace_size(
-      batch, n_q_heads, n_kv_heads, head_dim, max_seq_len, dtype, n_workgroups);
+  // Groups of fewer than four heads need fewer partials but more descriptors:
+  // a call that only fits the scratch with groups of four takes those.
+  int32_t heads = n_kv_heads > 0 ? heads_per_group(n_kv_heads) : kWaves;
+  int64_t need = workspace_size(batch, n_q_heads, n_kv_heads, head_dim, max_seq_len, dtype,
+                                n_workgroups, heads);
+  if (need > (int64_t)kScratchBytes && heads < kWaves) {
+    heads = kWaves;
+    need = workspace_size(batch, n_q_heads, n_kv_heads, head_dim, max_seq_len, dtype,
+                          n_workgroups, heads);
+  }
   if (need < 0) return (int)need;
   if ((uint64_t)need > kScratchBytes) return AEGKV_ERR_SCRATCH;
   if (batch == 0) return AEGKV_OK;
@@ -1754,32 +1808,17 @@ int aegkv_paged_decode_attention_noalloc(void* out, int64_t out_batch_stride, co
   return run_attention(out, out_batch_stride, q, q_batch_stride, key_cache, value_cache,
                        cache_block_stride, n_blocks, block_tables, max_blocks, nullptr, 0,
                        seq_lens, batch, max_seq_len, n_q_heads, n_kv_heads, head_dim,
-                       block_size, scale, dtype, n_workgroups, ws, kScratchBytes, stream);
+                       block_size, scale, dtype, n_workgroups, ws, kScratchBytes, stream,
+                       NewRows(), heads);
 }
 
 int64_t aegkv_paged_decode_attention_workspace_size(int32_t batch, int32_t n_q_heads,
                                                      int32_t n_kv_heads, int32_t head_dim,
                                                      int32_t max_seq_len, int32_t dtype,
                                                      int32_t n_workgroups) {
-  if (batch < 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_q_heads % n_kv_heads ||
-      n_workgroups < 0 || max_seq_len < 0)
-    return AEGKV_ERR_INVALID_ARG;
-  if (n_workgroups > kMaxWorkgroups) return AEGKV_ERR_UNSUPPORTED;
-  if ((head_dim != 64 && head_dim != 128 && head_dim != 256) ||
-      (dtype != AEGKV_DTYPE_BF16 && dtype != AEGKV_DTYPE_FP16) || n_q_heads / n_kv_heads > 16)
-    return AEGKV_ERR_UNSUPPORTED;
-  if (batch == 0) return 0;
-  const int32_t chunk = std::min(batch, kMaxBatch);
-  int n_wg = 0;
-  const int rc = workgroups_for(n_workgroups, &n_wg);
-  if (rc) return rc > 0 ? AEGKV_ERR_RUNTIME : rc;
-  const int32_t group = n_q_heads / n_kv_heads;
-  const int32_t n_groups = (n_kv_heads + kHeadsPerGroup - 1) / kHeadsPerGroup;
-  if (!positions_fit(chunk, ((int64_t)max_seq_len + kBlockSize - 1) / kBlockSize, n_groups, n_wg))
-    return AEGKV_ERR_UNSUPPORTED;
-  return workspace_layout(chunk, kHeadsPerGroup * group, head_dim, n_wg, n_groups).total;
+  return workspace_size(batch, n_q_heads, n_kv_heads, head_dim, max_seq_len, dtype, n_workgroups,
+                        heads_per_group(n_kv_heads));
 }
-
 
 int aegkv_paged_decode_attention(void* out, int64_t out_batch_stride, const void* q,
                                  int64_t q_batch_stride, const void* key_cache,
@@ -1849,9 +1888,11 @@ int64_t aegkv_paged_decode_plan_size(int32_t batch, int32_t n_kv_heads, int32_t 
   const int rc = workgroups_for(n_workgroups, &n_wg);
   if (rc) return rc > 0 ? AEGKV_ERR_RUNTIME : rc;
   const int64_t nblk_max = ((int64_t)max_seq_len + kBlockSize - 1) / kBlockSize;
-  const int32_t n_groups = (n_kv_heads + kHeadsPerGroup - 1) / kHeadsPerGroup;
-  if (!positions_fit(batch, nblk_max, n_groups, n_wg)) return AEGKV_ERR_UNSUPPORTED;
-  return plan_layout(batch, n_wg, nblk_max).total;
+  const int32_t heads = heads_per_group(n_kv_heads);
+  const int32_t n_ranges = n_wg * (kWaves / heads);
+  if (!positions_fit(batch, nblk_max, (n_kv_heads + heads - 1) / heads, n_ranges))
+    return AEGKV_ERR_UNSUPPORTED;
+  return plan_layout(batch, n_ranges, nblk_max).total;
 }
 
 int aegkv_paged_decode_plan(const int32_t* block_tables, int32_t max_blocks,
@@ -1869,7 +1910,9 @@ int aegkv_paged_decode_plan(const int32_t* block_tables, int32_t max_blocks,
   int n_wg = 0;
   int rc = workgroups_for(n_workgroups, &n_wg);
   if (rc) return rc;
-  const PlanLayout pl = plan_layout(batch, n_wg, nblk_max);
+  const int32_t heads = heads_per_group(n_kv_heads);
+  const int32_t n_ranges = n_wg * (kWaves / heads);
+  const PlanLayout pl = plan_layout(batch, n_ranges, nblk_max);
   uint8_t* pb = static_cast<uint8_t*>(plan);
   PlanArgs p;
   p.block_tables = block_tables;
@@ -1877,18 +1920,18 @@ int aegkv_paged_decode_plan(const int32_t* block_tables, int32_t max_blocks,
   p.seq_lens = seq_lens;
   p.batch = batch;
   p.max_seq_len = max_seq_len;
-  p.n_groups = (n_kv_heads + kHeadsPerGroup - 1) / kHeadsPerGroup;
-  p.n_wg = n_wg;
-  p.desc_per_seq = desc_per_sequence(batch, p.n_groups, n_wg) ? 1 : 0;
+  p.n_groups = (n_kv_heads + heads - 1) / heads;
+  p.n_ranges = n_ranges;
+  p.desc_per_seq = desc_per_sequence(batch, p.n_groups, n_ranges) ? 1 : 0;
   p.wg = reinterpret_cast<int32_t*>(pb + pl.wg);
   p.desc = reinterpret_cast<int4*>(pb + pl.desc);
   p.first = reinterpret_cast<int32_t*>(pb + pl.first);
   p.last = reinterpret_cast<int32_t*>(pb + pl.last);
   p.ids = reinterpret_cast<int32_t*>(pb + pl.ids);
   p.tags = reinterpret_cast<int32_t*>(pb + pl.tags);
-  const int64_t work = std::max<int64_t>((int64_t)n_wg * 64, (int64_t)batch * nblk_max);
+  const int64_t work = std::max<int64_t>((int64_t)n_ranges * 64, (int64_t)batch * nblk_max);
   const int grid = (int)std::max<int64_t>(1, std::min<int64_t>(1024, (work + 255) / 256));
-  hipLaunchKernelGGL(decode_plan_kernel, dim3(grid), dim3(64 * kHeadsPerGroup),
+  hipLaunchKernelGGL(decode_plan_kernel, dim3(grid), dim3(64 * kWaves),
                      (size_t)(3 * batch + 2) * sizeof(int32_t), (hipStream_t)stream, p);
   AEGKV_HIP_TRY(hipGetLastError());
   return AEGKV_OK;

@@ -945,3 +945,44 @@ def test_merge_shared_by_workgroups(device, Hq, Hkv, D, lens, nwg):
                                     ko.bits_to_float(vc, "bf16"), padded, lens, scale)
     _check(to_bits(one), ref, "bf16")
     assert np.array_equal(to_bits(one), to_bits(two))
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(3, 3, 128), (14, 2, 128), (10, 10, 64), (7, 1, 128),
+                                      (5, 5, 256), (66, 66, 64)])
+@pytest.mark.parametrize("nwg", [0, 1, 5])
+def test_kv_head_counts_not_of_four(device, Hq, Hkv, D, nwg):
+    """Head counts that make groups of two and one kv heads (a workgroup then
+    holds two or four ranges), and one above the bound that keeps groups of
+    four with idle waves: planned, unplanned and appending calls."""
+    lens = [1, 16, 33, 700, 0, 129, 1500]
+    rng = np.random.default_rng(Hq + nwg)
+    lens, tables, padded, q, kc, vc = _setup(rng, lens, Hq, Hkv, D, "fp16")
+    scale = 1.0 / math.sqrt(D)
+    dev = lambda x: to_device_bits(x, "fp16", device)  # noqa: E731
+    bt = torch.from_numpy(padded).to(device)
+    sl = torch.from_numpy(lens.astype(np.int32)).to(device)
+    ml = int(lens.max())
+    dq, dk, dv = dev(q), dev(kc), dev(vc)
+    key = dev(random_bits(rng, (len(lens), Hkv, D), "fp16"))
+    val = dev(random_bits(rng, (len(lens), Hkv, D), "fp16"))
+    one = A.paged_decode_attention(dq, dk, dv, bt, sl, scale, ml, n_workgroups=nwg)
+    ref = ko.paged_decode_attention(ko.bits_to_float(q, "fp16"), ko.bits_to_float(kc, "fp16"),
+                                    ko.bits_to_float(vc, "fp16"), padded, lens, scale)
+    _check(to_bits(one), ref, "fp16")
+    plan = A.DecodePlan(bt, sl, ml, Hkv, nwg)
+    two = A.paged_decode_attention(dq, dk, dv, None, None, scale, ml, n_workgroups=nwg, plan=plan)
+    assert np.array_equal(to_bits(one), to_bits(two))
+    rows = [b for b in range(len(lens)) if lens[b] > 0]
+    slots = np.full(len(lens), -1, dtype=np.int64)
+    for b in rows:
+        p = int(lens[b]) - 1
+        slots[b] = tables[b][p // 16] * 16 + p % 16
+    k2, v2 = dk.clone(), dv.clone()
+    A.reshape_and_cache_flash(key, val, k2, v2, torch.from_numpy(slots).to(device))
+    want = A.paged_decode_attention(dq, k2, v2, bt, sl, scale, ml, n_workgroups=nwg)
+    for pl in (None, plan):
+        k3, v3 = dk.clone(), dv.clone()
+        got = A.paged_decode_attention(dq, k3, v3, None if pl else bt, None if pl else sl, scale,
+                                       ml, n_workgroups=nwg, plan=pl, key=key, value=val)
+        assert np.array_equal(to_bits(got), to_bits(want))
+        assert np.array_equal(to_bits(k3), to_bits(k2)) and np.array_equal(to_bits(v3), to_bits(v2))
