@@ -45,22 +45,26 @@
 // is faster: 4 x 2048 cache-cold 174.0 against 181.0 us, 2 x 4096 269.5
 // against 303.7 us, 1 x 8192 544.7 against 627.3 us.)
 //
-// Work order, both kernels: the (sequence, query head) units, in that order
-// (so the query heads of one kv head are neighbours), are split into kXcds
-// contiguous runs, one per XCD: the hardware deals workgroup i to XCD
-// i % kXcds, and workgroup i = s * kXcds + x takes the s-th job of XCD x's
-// run.  Every query tile of a unit then runs on one XCD, whose L2 keeps that
-// sequence's K and V for all of them.  When the units do not divide evenly
-// over the XCDs and each CU has several tiles to run, a unit's tiles are
-// dealt as S interleaved slices instead (slices_per_unit), so every XCD
-// holds the same number of slices.  A ragged batch (by the host bound) deals
-// its units round-robin over the XCDs, so no XCD holds only the longest
-// prompts.  Within an XCD the jobs run with the
-// query tile slowest, in decreasing order, so the most expensive tiles (the
-// last of each sequence) are dispatched first.  (A persistent grid dealing the
-// same jobs in snake order measured 5% slower on 4 x 2048 tokens and 60%
-// slower on ragged batches, whose short sequences leave most high-tile jobs
-// empty.)
+// Wave units, both kernels: the work of a (sequence, kv head) pair is cut into
+// units of 32 queries of one query head, unit u = query block u / G of the
+// head u % G of the kv head's G; a workgroup's waves take consecutive units.
+// They share the pair's K and V tiles, and since the heads of one query block
+// are neighbours, a causal workgroup's waves need (almost) the same keys and a
+// short or ragged prompt leaves no wave without queries but its last.  (A
+// workgroup of 128 or 256 queries of one head idled its early waves on the
+// diagonal tiles and its late ones past the end: 48 prompts of 25-766 tokens
+// 111.1 -> 94.0 us, 4 x 2048 of 28/4 heads 151.5 -> 142.4.)
+//
+// Work order, both kernels: a job is a tile of a pair's units, and the jobs
+// run with the tile index slowest, in decreasing order, so the most expensive
+// tiles (the last of each sequence) are dispatched first; within a tile index
+// the pairs follow each other, kv heads fastest.  The hardware deals workgroup
+// i to XCD i % 8: with a multiple of 8 pairs of one length, XCD x runs every
+// tile of the x-th eighth of the pairs, whose K and V its L2 keeps (1 x 4096
+// tokens of 40 heads: 193.5 us against 197.4 with the pairs dealt in turn), and
+// fewer pairs spread evenly over the XCDs.  Prompts of different lengths: each wave finds job i
+// among the tiles that exist (pick_job), so no workgroup is launched for an
+// empty tile (48 prompts of 25-766 tokens: 5900 of 9200 workgroups were).
 #include <algorithm>
 #include <cmath>
 
@@ -87,12 +91,13 @@ constexpr float kPfRescaleSlack = 8.f;
 constexpr int kLongPrompt = 1536;            // longer prompts take the ping-pong kernel
 // short-prompt kernel: four waves, 128 queries, V^T staged transposed
 constexpr int kShortThreads = 256;
-constexpr int kShortQTile = 128;
+constexpr int kShortWaves = kShortThreads / 64;
 constexpr int kVtPitch = kPfKTile * 2 + 16;  // bytes per row of V^T in LDS
 // ping-pong kernel: eight waves, 256 queries
 constexpr int kLongWaves = 8;
 constexpr int kLongThreads = 64 * kLongWaves;
-constexpr int kLongQTile = 32 * kLongWaves;
+constexpr int kUnitQ = 32;       // queries of a wave unit
+constexpr int kCompactSets = 4;  // 64-sequence sets a wave searches for its job
 
 template <int DT>
 struct PfOps;
@@ -148,10 +153,10 @@ struct PrefillArgs {
   int64_t q_tok_b, k_tok_b, v_tok_b, o_tok_b;  // byte strides per token
   const int32_t* cu_seqlens;                   // [batch + 1], device
   int64_t total_tokens;
-  int32_t batch, n_q_heads, group, max_seqlen, n_qtiles, causal;
-  int32_t n_units;                             // batch * n_q_heads
-  int32_t slices;                              // interleaved tile slices per unit
-  int32_t interleave;                          // slices dealt round-robin over the XCDs
+  int32_t batch, n_kv_heads, group, max_seqlen, causal;
+  int32_t n_pairs;                             // batch * n_kv_heads
+  int32_t n_tiles;                             // tiles of a pair of max_seqlen tokens
+  int32_t compact;                             // jobs numbered over existing tiles only
   float scale_log2;                            // softmax scale * log2(e), > 0
 };
 
@@ -291,51 +296,99 @@ struct WaveState {
   }
 };
 
-// Uniform job of workgroup blockIdx.x for query tiles of qtile queries:
-// returns false when the tile is empty.  Slice v = unit * S + r holds the
-// unit's tiles r, r + S, ...; XCD x holds c slices, the run [v0, v0 + c) or,
-// interleaved, slices x, x + kXcds, ...; its s-th job is the (s / c)-th
-// largest tile of its (s % c)-th slice.
-__device__ __forceinline__ bool pick_job(const PrefillArgs& a, int qtile, int& h, int64_t& s0,
-                                         int& len, int& q0) {
-  const int x = (int)(blockIdx.x % kXcds), sj = (int)(blockIdx.x / kXcds);
-  const int S = a.slices;
-  const int64_t n_sl = (int64_t)a.n_units * S;
-  int c, v;
-  if (a.interleave) {
-    c = (int)((n_sl - x + kXcds - 1) / kXcds);
-    if (c <= 0) return false;
-    v = x + kXcds * (sj % c);
-  } else {
-    const int v0 = (int)(n_sl * x / kXcds);
-    c = (int)(n_sl * (x + 1) / kXcds) - v0;
-    if (c == 0) return false;
-    v = v0 + sj % c;
+// The clamped token range of sequence b.
+__device__ __forceinline__ void seq_range(const PrefillArgs& a, int b, int& s0, int& len) {
+  const int64_t c0 = a.cu_seqlens[b], c1 = a.cu_seqlens[b + 1];
+  const int64_t lo = min(max(c0, (int64_t)0), a.total_tokens);
+  const int64_t hi = min(max(c1, lo), a.total_tokens);
+  s0 = (int)lo;  // total_tokens may exceed it, cu_seqlens' values do not
+  len = (int)min(hi - lo, (int64_t)a.max_seqlen);
+}
+
+// Sum over the wave's lanes, uniform.
+__device__ __forceinline__ int wave_sum(int x) {
+  x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);  // row_shr 1
+  x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);  // row_shr 2
+  x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);  // row_shr 4
+  x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);  // row_shr 8
+  x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, true);  // row_bcast 15, rows 1 and 3
+  x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, true);  // row_bcast 31, rows 2 and 3
+  return __builtin_amdgcn_readlane(x, 63);
+}
+
+// The job of workgroup blockIdx.x of W waves (uniform): sequence range, kv
+// head and first unit.  Returns false when the tile is empty or there are
+// fewer jobs.
+template <int W>
+__device__ __forceinline__ bool pick_job(const PrefillArgs& a, int& kvh, int& s0, int& len,
+                                         int& u0) {
+  const uint32_t i = blockIdx.x;
+  const int G = a.group, H = a.n_kv_heads;
+  auto tiles_of = [&](int n) { return ((n + kUnitQ - 1) / kUnitQ * G + W - 1) / W; };
+  if (!a.compact) {  // every tile of the bound: tile n_tiles - 1 of each pair first
+    const int k = (int)(i / (uint32_t)a.n_pairs);
+    int r = (int)(i - (uint32_t)k * a.n_pairs);
+    if (a.n_pairs % kXcds == 0) r = r % kXcds * (a.n_pairs / kXcds) + r / kXcds;
+    kvh = r % H;
+    seq_range(a, r / H, s0, len);
+    const int tile = a.n_tiles - 1 - k;
+    u0 = tile * W;
+    return tile < tiles_of(len);
   }
-  const int k = sj / c;
-  const int unit = v / S, r = v - unit * S;
-  const int m = (a.n_qtiles - r + S - 1) / S;  // tiles in slice r
-  if (k >= m) return false;
-  const int tile = r + S * (m - 1 - k);
-  const int b = unit / a.n_q_heads;
-  h = unit % a.n_q_heads;
-  int64_t s1 = a.cu_seqlens[b + 1];
-  s0 = a.cu_seqlens[b];
-  s0 = min(max(s0, (int64_t)0), a.total_tokens);
-  s1 = min(max(s1, s0), a.total_tokens);
-  len = (int)min(s1 - s0, (int64_t)a.max_seqlen);
-  q0 = tile * qtile;
-  return q0 < len;
+  const int lane = threadIdx.x & 63;
+  int st[kCompactSets], ln[kCompactSets], t[kCompactSets];
+#pragma unroll
+  for (int k = 0; k < kCompactSets; ++k) {
+    const int b = 64 * k + lane;
+    st[k] = ln[k] = 0;
+    if (64 * k < a.batch) seq_range(a, min(b, a.batch - 1), st[k], ln[k]);
+    t[k] = b < a.batch ? tiles_of(ln[k]) : 0;
+  }
+  auto jobs_from = [&](int tile) -> uint32_t {  // jobs of tile index >= tile
+    int x = 0;
+#pragma unroll
+    for (int k = 0; k < kCompactSets; ++k) x += max(t[k] - tile, 0);
+    return (uint32_t)wave_sum(x) * (uint32_t)H;
+  };
+  if (jobs_from(0) <= i) return false;
+  int lo = 0, hi = a.n_tiles;  // jobs_from(lo) > i >= jobs_from(hi)
+  uint32_t after = 0;          // jobs_from(hi)
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) >> 1;
+    const uint32_t n = jobs_from(mid);
+    if (n > i) lo = mid;
+    else { hi = mid; after = n; }
+  }
+  int rank = (int)((i - after) / (uint32_t)H);
+  kvh = (int)((i - after) - (uint32_t)rank * H);
+  u0 = lo * W;
+  // the rank-th sequence with a tile `lo`
+  s0 = len = 0;
+#pragma unroll
+  for (int k = 0; k < kCompactSets; ++k) {
+    const uint64_t mask = __builtin_amdgcn_ballot_w64(t[k] > lo);
+    const int c = __builtin_popcountll(mask);
+    if (rank >= 0 && rank < c) {
+      const int at = (int)__builtin_amdgcn_mbcnt_hi(
+          (uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
+      const uint64_t hit = __builtin_amdgcn_ballot_w64(t[k] > lo && at == rank);
+      const int src = __builtin_ctzll(hit);
+      s0 = __builtin_amdgcn_readlane(st[k], src);
+      len = __builtin_amdgcn_readlane(ln[k], src);
+    }
+    rank -= c;
+  }
+  return true;
 }
 
 // ---------------------------------------------------------------- short prompts
-// Queries [q0, q0 + 128) of head h of the sequence at token s0 with len
+// Units [u0, u0 + 4) of kv head kvh of the sequence at token s0 with len
 // tokens; K and V tiles staged through registers, two stages each in LDS (V
 // transposed, the 4-key quads of every 16 keys in the order 0, 2, 1, 3, so each
 // P.V operand is one 16-byte LDS read).
 template <int DT, int D>
-__device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds, int h, int64_t s0,
-                                             int len, int q0) {
+__device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds, int kvh,
+                                             int64_t s0, int len, int u0) {
   using E = PfOps<DT>;
   using W = WaveState<DT, D>;
   constexpr int KPITCH = D * 2 + 16;            // bytes per K row in LDS
@@ -346,15 +399,15 @@ __device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds,
   constexpr int KRPP = kShortThreads / CPR;     // K rows staged per pass
   constexpr int KPASS = kPfKTile / KRPP;
   constexpr int VTHREADS = (kPfKTile / 4) * CPR;  // (4-key quad, chunk) pairs
-  const int kvh = h / a.group;
-  const int kv_end = a.causal ? min(len, q0 + kShortQTile) : len;
+  const int kv_end = a.causal ? min(len, (u0 + kShortWaves - 1) / a.group * kUnitQ + kUnitQ) : len;
   const int n_kt = (kv_end + kPfKTile - 1) / kPfKTile;
 
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);  // uniform: the tile tests below branch
   const int col = lane & 31, hh = lane >> 5;
-  const int qi = q0 + 32 * w + col;  // this lane's query, relative to the sequence
-  const int wq0 = q0 + 32 * w;       // the wave's first query
+  const int h = kvh * a.group + (u0 + w) % a.group;
+  const int wq0 = (u0 + w) / a.group * kUnitQ;  // the wave's first query
+  const int qi = wq0 + col;                     // this lane's query, relative to the sequence
   W st;
   st.init(a, h, s0, len, qi, hh);
 
@@ -446,7 +499,7 @@ __device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds,
       load_k(kt + 1);
       load_v(kt + 1);
     }
-    if (!a.causal || kt * kPfKTile <= wq0 + 31) {
+    if (wq0 < len && (!a.causal || kt * kPfKTile <= wq0 + 31)) {
       f32x16 sc[2];
       u32x4 pb[4];
       st.template qk<KPITCH, 0>(lds + (kt & 1) * K_BYTES + col * KPITCH + 16 * hh, sc);
@@ -469,18 +522,17 @@ __global__ __launch_bounds__(kShortThreads, 2) void prefill_short_kernel(Prefill
   constexpr int V_BYTES = D * kVtPitch;
   // two K stages, then two V^T stages
   __shared__ __align__(16) uint8_t lds[2 * K_BYTES + 2 * V_BYTES];
-  int h, len, q0;
-  int64_t s0;
-  if (!pick_job(a, kShortQTile, h, s0, len, q0)) return;  // uniform, before any barrier
-  attend_short<DT, D>(a, lds, h, s0, len, q0);
+  int kvh, s0, len, u0;
+  if (!pick_job<kShortWaves>(a, kvh, s0, len, u0)) return;  // uniform, before any barrier
+  attend_short<DT, D>(a, lds, kvh, s0, len, u0);
 }
 
 // ----------------------------------------------------------------- long prompts
-// Queries [q0, q0 + 256) of head h of the sequence at token s0 with len
+// Units [u0, u0 + 8) of kv head kvh of the sequence at token s0 with len
 // tokens, ping-pong between the workgroup's halves.
 template <int DT, int D>
-__device__ __forceinline__ void attend_long(const PrefillArgs& a, uint8_t* lds, int h, int64_t s0,
-                                            int len, int q0) {
+__device__ __forceinline__ void attend_long(const PrefillArgs& a, uint8_t* lds, int kvh,
+                                            int64_t s0, int len, int u0) {
   using E = PfOps<DT>;
   using W = WaveState<DT, D>;
   constexpr int KPITCH = D * 2 + 16;            // bytes per K row in LDS
@@ -495,16 +547,16 @@ __device__ __forceinline__ void attend_long(const PrefillArgs& a, uint8_t* lds, 
   constexpr int NK = (CK + kLongWaves - 1) / kLongWaves;
   constexpr int NV = (CV + kLongWaves - 1) / kLongWaves;
   constexpr uint32_t kPad = 0xFFFFFFF0u;        // an offset out of every range
-  const int kvh = h / a.group;
-  const int kv_end = a.causal ? min(len, q0 + kLongQTile) : len;
+  const int kv_end = a.causal ? min(len, (u0 + kLongWaves - 1) / a.group * kUnitQ + kUnitQ) : len;
   const int n_kt = (kv_end + kPfKTile - 1) / kPfKTile;
 
   const int t = threadIdx.x, lane = t & 63;
   const int w = __builtin_amdgcn_readfirstlane(t >> 6);  // uniform: the tile tests below branch
   const int half = w >> 2;           // 0: waves 0-3, 1: waves 4-7 (one phase later)
   const int col = lane & 31, hh = lane >> 5;
-  const int qi = q0 + 32 * w + col;  // this lane's query, relative to the sequence
-  const int wq0 = q0 + 32 * w;       // the wave's first query
+  const int h = kvh * a.group + (u0 + w) % a.group;
+  const int wq0 = (u0 + w) / a.group * kUnitQ;  // the wave's first query
+  const int qi = wq0 + col;                     // this lane's query, relative to the sequence
   // the wave's last key tile: causal waves stop at their last query's tile; a
   // wave past the end of the sequence attends to nothing (-1)
   const int jw = wq0 >= len ? -1
@@ -667,38 +719,9 @@ __global__ __launch_bounds__(kLongThreads) void prefill_long_kernel(PrefillArgs 
   constexpr int V_BYTES = kPfKTile * (D * 2 + 64);
   // two K stages, then two V stages
   __shared__ __align__(16) uint8_t lds[2 * K_BYTES + 2 * V_BYTES];
-  int h, len, q0;
-  int64_t s0;
-  if (!pick_job(a, kLongQTile, h, s0, len, q0)) return;  // uniform, before any barrier
-  attend_long<DT, D>(a, lds, h, s0, len, q0);
-}
-
-// Tile slices per unit.  With n_units not a multiple of kXcds, whole units
-// leave some XCDs a unit more than others (1 x 8192 tokens of 28 heads: four
-// XCDs hold 4 units, four hold 3, and the latter idle an eighth of the
-// time).  S interleaved slices per unit, the smallest S with S * n_units a
-// multiple of kXcds, even that out.  That pays only when the heaviest XCD's
-// CUs take at least three tiles each: with fewer, its largest tiles set the
-// end whatever the split, and the split unit's K/V fills two XCDs' L2.
-// (Measured, same process: 1 x 8192 505.9 -> 481.8 us, 1 x 16384 2099 ->
-// 1940 us; 1 x 4096, at two tiles per CU, 140.0 -> 145.8 us without the
-// threshold.)
-int slices_per_unit(int64_t n_units, int64_t n_qtiles, int cus_per_xcd) {
-  int64_t g = kXcds;
-  for (int64_t u = n_units % kXcds; u != 0;) {
-    const int64_t t = g % u;
-    g = u;
-    u = t;
-  }
-  const int64_t S = std::min<int64_t>(kXcds / g, n_qtiles);
-  if (S <= 1 || (n_units + kXcds - 1) / kXcds * n_qtiles < 3 * (int64_t)cus_per_xcd) return 1;
-  return (int)S;
-}
-
-// kXcds runs of at most ceil(S * n_units / kXcds) slices of at most
-// ceil(n_qtiles / S) tiles
-int64_t grid_size(int64_t n_units, int64_t n_qtiles, int S) {
-  return kXcds * ((n_qtiles + S - 1) / S) * ((S * n_units + kXcds - 1) / kXcds);
+  int kvh, s0, len, u0;
+  if (!pick_job<kLongWaves>(a, kvh, s0, len, u0)) return;  // uniform, before any barrier
+  attend_long<DT, D>(a, lds, kvh, s0, len, u0);
 }
 
 template <int DT, int D>
@@ -742,22 +765,31 @@ int aegkv_varlen_prefill_attention(void* out, int64_t out_token_stride, const vo
   if (!aligned16(out) || !aligned16(q) || !aligned16(k) || !aligned16(v) ||
       q_token_stride % 8 || k_token_stride % 8 || v_token_stride % 8 || out_token_stride % 8)
     return AEGKV_ERR_MISALIGNED;
-  const int64_t n_units = (int64_t)n_q_heads * batch;
   const bool long_prompts = max_seqlen > kLongPrompt;
-  const int qtile = long_prompts ? kLongQTile : kShortQTile;
-  const int64_t n_qtiles = ((int64_t)max_seqlen + qtile - 1) / qtile;
-  if (kXcds * n_units * n_qtiles > INT32_MAX) return AEGKV_ERR_UNSUPPORTED;
+  const int waves = long_prompts ? kLongWaves : kShortWaves;
+  const int group = n_q_heads / n_kv_heads;
+  const int64_t n_pairs = (int64_t)n_kv_heads * batch;
+  const int64_t max_units = ((int64_t)max_seqlen + kUnitQ - 1) / kUnitQ * group;
+  const int64_t n_tiles = (max_units + waves - 1) / waves;
+  // a bound of the jobs (8 x query heads x whole tiles), well below 2^31
+  const int64_t q_tiles = (max_units / group + waves - 1) / waves;
+  if (8 * (int64_t)n_q_heads * batch * q_tiles > INT32_MAX) return AEGKV_ERR_UNSUPPORTED;
   // the long kernel addresses K and V rows by 32-bit byte offsets within a
   // sequence, up to one key tile past its end
   if (long_prompts && ((int64_t)max_seqlen + kPfKTile) *
                               std::max(k_token_stride, v_token_stride) * 2 >
                           (int64_t)UINT32_MAX)
     return AEGKV_ERR_UNSUPPORTED;
-  DeviceState* ds = nullptr;
-  if (int rc = current_device_state(&ds)) return rc;
-  const int slices = slices_per_unit(n_units, n_qtiles, std::max(1, ds->num_cu / kXcds));
-  const int64_t grid = grid_size(n_units, n_qtiles, slices);
-  if (grid > INT32_MAX) return AEGKV_ERR_UNSUPPORTED;
+  // Job numbers over the existing tiles only, unless the lengths are all the
+  // bound (nothing to skip) or there are more than a wave searches.  The sum of
+  // the tiles is bounded by the tokens, plus a part-filled unit and tile per
+  // sequence.
+  const bool compact = total_tokens < (int64_t)batch * max_seqlen && batch <= 64 * kCompactSets;
+  int64_t grid = n_pairs * n_tiles;
+  if (compact) {
+    const int64_t units = (total_tokens / kUnitQ + batch) * group;
+    grid = std::min(grid, (units / waves + batch) * n_kv_heads);
+  }
 
   PrefillArgs a;
   a.q = static_cast<const uint8_t*>(q);
@@ -771,20 +803,12 @@ int aegkv_varlen_prefill_attention(void* out, int64_t out_token_stride, const vo
   a.cu_seqlens = cu_seqlens;
   a.total_tokens = total_tokens;
   a.batch = batch;
-  a.n_q_heads = n_q_heads;
-  a.group = n_q_heads / n_kv_heads;
+  a.n_kv_heads = n_kv_heads;
+  a.group = group;
   a.max_seqlen = max_seqlen;
-  a.n_qtiles = (int32_t)n_qtiles;
-  a.n_units = (int32_t)n_units;
-  a.slices = slices;
-  // Prompts of different lengths: contiguous runs would give each XCD whole
-  // prompts (8 prompts of 28 heads: one per XCD, the longest setting the
-  // end), so the units are dealt round-robin instead.  That spreads one kv
-  // head's query heads over several L2s, which costs uniform batches 1-4%,
-  // so it is kept for batches the host bound shows to be ragged (fewer
-  // tokens than 90% of batch x max_seqlen).  Same process, 8 prompts of
-  // 77-2048 tokens: 281.7 -> 149.6 us.
-  a.interleave = total_tokens * 10 < (int64_t)batch * max_seqlen * 9 ? 1 : 0;
+  a.n_pairs = (int32_t)n_pairs;
+  a.n_tiles = (int32_t)n_tiles;
+  a.compact = compact ? 1 : 0;
   a.causal = causal ? 1 : 0;
   a.scale_log2 = scale * 1.4426950408889634f;
   const uint32_t g32 = (uint32_t)grid;

@@ -291,3 +291,26 @@ def test_wrapper_rejects_unsupported_options():
     with pytest.raises(AegkvError):
         A.varlen_prefill_attention(q[:, :, :32].contiguous(), k[:, :, :32].contiguous(),
                                    v[:, :, :32].contiguous(), cu_t, 10, 0.1)
+
+
+@pytest.mark.parametrize("Hq,Hkv", [(7, 1), (6, 2), (4, 4)])
+@pytest.mark.parametrize("top", [130, 1600])  # the four-wave and the ping-pong kernel
+@pytest.mark.parametrize("causal", [True, False])
+def test_jobs_over_existing_tiles(Hq, Hkv, top, causal):
+    """The numbering of jobs over the tiles that exist (batches of up to 256
+    sequences) against the one over the bound's (above), bit for bit: the first
+    256 sequences alone, then beside a 257th; empty sequences, one query, edges
+    of the 32-query units, tiles shared by the heads of two query blocks."""
+    rng = np.random.default_rng(Hq + top)
+    lens = rng.integers(0, 100, 257)
+    lens[[0, 3, 100, 255]] = [top, 0, 1, 33]
+    cu, q, k, v = _packed(lens.tolist(), Hq, Hkv, 64, torch.bfloat16, 5)
+    cu_t = torch.from_numpy(cu).cuda()
+    all_ = A.varlen_prefill_attention(q, k, v, cu_t, top, 0.125, causal)
+    n = int(cu[256])
+    first = A.varlen_prefill_attention(q[:n], k[:n], v[:n], cu_t[:257], top, 0.125, causal)
+    few = A.varlen_prefill_attention(q[:int(cu[8])], k[:int(cu[8])], v[:int(cu[8])], cu_t[:9], top,
+                                     0.125, causal)
+    assert torch.equal(first.view(torch.int16), all_[:n].view(torch.int16))
+    assert torch.equal(few.view(torch.int16), all_[:int(cu[8])].view(torch.int16))
+    _check(few, q, k, v, cu[:9], 0.125, causal, torch.bfloat16, int(cu[8]))
