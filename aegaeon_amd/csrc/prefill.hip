@@ -36,10 +36,9 @@
 // (buffer loads with the LDS bit, no registers), V untransposed, and the
 // P.V operands are read with gfx950's transposing LDS reads.
 //
-// Short prompts: two workgroups of four waves per CU, each taking 128 queries;
-// K and V are staged through registers (V transposed on the way into LDS) and
-// the two workgroups overlap each other's softmax and matrix work unordered.
-// (With short prompts the ping-pong workgroup's start-up and its larger
+// Short prompts: three workgroups of four waves per CU that overlap each
+// other's latencies, softmax and matrix work unordered; K and V reach LDS the
+// same way.  (With short prompts the ping-pong workgroup's start-up and its larger
 // causal diagonal cost more than the phase overlap gains: 8 x 1024 tokens
 // 112.6 against 109.0 us, 16 x 512 90.1 against 78.5 us; from 2048 tokens on it
 // is faster: 4 x 2048 cache-cold 174.0 against 181.0 us, 2 x 4096 269.5
@@ -89,11 +88,10 @@ constexpr int kXcds = 8;                     // XCDs of an MI355X (gfx950)
 constexpr int kPfKTile = 64;                 // keys per step
 constexpr float kPfRescaleSlack = 8.f;
 constexpr int kLongPrompt = 1536;            // longer prompts take the ping-pong kernel
-// short-prompt kernel: four waves, 128 queries, V^T staged transposed
+// short-prompt kernel: four waves
 constexpr int kShortThreads = 256;
 constexpr int kShortWaves = kShortThreads / 64;
-constexpr int kVtPitch = kPfKTile * 2 + 16;  // bytes per row of V^T in LDS
-// ping-pong kernel: eight waves, 256 queries
+// ping-pong kernel: eight waves
 constexpr int kLongWaves = 8;
 constexpr int kLongThreads = 64 * kLongWaves;
 constexpr int kUnitQ = 32;       // queries of a wave unit
@@ -135,14 +133,6 @@ struct PfOps<AEGKV_DTYPE_FP16> {
 // costs a few canonicalising v_max_f32 (0-3% per call).
 __device__ __forceinline__ float max3(float a, float b, float c) {
   return __builtin_fmaxf(__builtin_fmaxf(a, b), c);
-}
-
-// {lo16(a), lo16(b)} and {hi16(a), hi16(b)} (v_perm_b32: src1 = bytes 0-3)
-__device__ __forceinline__ uint32_t pack_lo(uint32_t a, uint32_t b) {
-  return __builtin_amdgcn_perm(b, a, 0x05040100u);
-}
-__device__ __forceinline__ uint32_t pack_hi(uint32_t a, uint32_t b) {
-  return __builtin_amdgcn_perm(b, a, 0x07060302u);
 }
 
 struct PrefillArgs {
@@ -383,22 +373,29 @@ __device__ __forceinline__ bool pick_job(const PrefillArgs& a, int& kvh, int& s0
 
 // ---------------------------------------------------------------- short prompts
 // Units [u0, u0 + 4) of kv head kvh of the sequence at token s0 with len
-// tokens; K and V tiles staged through registers, two stages each in LDS (V
-// transposed, the 4-key quads of every 16 keys in the order 0, 2, 1, 3, so each
-// P.V operand is one 16-byte LDS read).
+// tokens.  K and V tiles go from HBM straight into LDS (loads with the LDS bit)
+// and V's operands are read with the transposing LDS reads, so a workgroup
+// holds 48 KiB of LDS (two K stages, one V stage) and no staging registers,
+// and three of them share a CU: a prompt of a few key tiles is a chain of
+// latencies (job, first tiles, stores), which only other workgroups hide.
+// (Two per CU with K and V staged through registers and V transposed on the way
+// into LDS: 48 prompts of 25-766 tokens 94.0 us, 8 x 1024 95.5, 16 x 512 69.0;
+// this 84.5, 87.6, 62.8.)
+// Rows are stored unpadded with their 16-byte chunks permuted by the row
+// (the loads pick the chunk, the LDS position is the lane's): K chunk c of row
+// r at c ^ (r % 16) at D = 128, V chunk c at c ^ 4 (r % 4), so the 16 rows of a
+// K read and the 4 rows of a transposing V read hit distinct banks.
 template <int DT, int D>
 __device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds, int kvh,
                                              int64_t s0, int len, int u0) {
   using E = PfOps<DT>;
   using W = WaveState<DT, D>;
-  constexpr int KPITCH = D * 2 + 16;            // bytes per K row in LDS
-  constexpr int K_BYTES = kPfKTile * KPITCH;
-  constexpr int V_BYTES = D * kVtPitch;
+  constexpr int RB = D * 2;                     // bytes per row
+  constexpr int T_BYTES = kPfKTile * RB;        // bytes per tile
   constexpr int DB = W::DB;
   constexpr int CPR = D / 8;                    // 16-byte chunks per row
-  constexpr int KRPP = kShortThreads / CPR;     // K rows staged per pass
-  constexpr int KPASS = kPfKTile / KRPP;
-  constexpr int VTHREADS = (kPfKTile / 4) * CPR;  // (4-key quad, chunk) pairs
+  constexpr int RPI = 64 / CPR;                 // rows per load instruction
+  constexpr int NI = kPfKTile / (RPI * kShortWaves);  // load instructions per wave and tile
   const int kv_end = a.causal ? min(len, (u0 + kShortWaves - 1) / a.group * kUnitQ + kUnitQ) : len;
   const int n_kt = (kv_end + kPfKTile - 1) / kPfKTile;
 
@@ -408,120 +405,107 @@ __device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds,
   const int h = kvh * a.group + (u0 + w) % a.group;
   const int wq0 = (u0 + w) / a.group * kUnitQ;  // the wave's first query
   const int qi = wq0 + col;                     // this lane's query, relative to the sequence
+
+  // Load instruction ii of wave w covers rows RPI (w + 4 ii) .. of a tile, lane
+  // l the chunk stored at byte 16 l of them; the permutations depend on the
+  // lane and wave only (rows 4 RPI apart permute alike).
+  const int lrow = RPI * w + lane / CPR, lpos = lane % CPR;
+  const int kch = D == 128 ? lpos ^ (lrow & 15) : lpos ^ ((lrow >> 1) & 7);
+  const int vch = D == 128 ? lpos ^ ((lrow & 3) << 2) : lpos ^ (((lrow >> 1) & 1) << 2);
+  const uint8_t* kbase = a.k + s0 * a.k_tok_b + (int64_t)kvh * RB + kch * 16;
+  const uint8_t* vbase = a.v + s0 * a.v_tok_b + (int64_t)kvh * RB + vch * 16;
+  auto dma = [&](const uint8_t* base, int64_t tok_b, int kt, uint8_t* stage) {
+#pragma unroll
+    for (int ii = 0; ii < NI; ++ii) {
+      // rows past the sequence re-read its last one: their scores are masked,
+      // their weights 0
+      const int row = min(kt * kPfKTile + lrow + kShortWaves * RPI * ii, len - 1);
+      __builtin_amdgcn_global_load_lds(
+          (const __attribute__((address_space(1))) void*)(base + row * tok_b),
+          (lds_void*)(stage + (w + kShortWaves * ii) * 1024), 16, 0, 0);
+    }
+  };
+  auto dma_k = [&](int kt) { dma(kbase, a.k_tok_b, kt, lds + (kt & 1) * T_BYTES); };
+  auto dma_v = [&](int kt) { dma(vbase, a.v_tok_b, kt, lds + 2 * T_BYTES); };
+  dma_k(0);
   W st;
   st.init(a, h, s0, len, qi, hh);
+  dma_v(0);
 
-  // staging: K row kr + KRPP p, chunk kc; V keys 4 vq .. 4 vq + 3, chunk vc
-  const uint8_t* kbase = a.k + s0 * a.k_tok_b + (int64_t)kvh * D * 2;
-  const uint8_t* vbase = a.v + s0 * a.v_tok_b + (int64_t)kvh * D * 2;
-  const int kc = t % CPR, kr = t / CPR;
-  const int vq = t % (kPfKTile / 4), vc = t / (kPfKTile / 4);
-  // position of the quad in the stored key order (quads 0, 2, 1, 3 of 16 keys)
-  const int vpos = 16 * (vq >> 2) + 4 * (((vq & 1) << 1) | ((vq >> 1) & 1));
-  const uint32_t koff = (uint32_t)(kr * a.k_tok_b) + kc * 16;
-  const uint32_t voff = (uint32_t)(4 * vq * a.v_tok_b) + vc * 16;
-  u32x4 kreg[KPASS], vreg[4];
-
-  auto load_k = [&](int kt) {
-    const int r0 = kt * kPfKTile;
-    if (r0 + kPfKTile <= len) {  // whole tile inside the sequence (uniform)
-      const uint8_t* kb = kbase + r0 * a.k_tok_b;
+  // K operand: row col (+ 32 sb), chunk 2 ks + hh
+  const int kx = D == 128 ? (hh ^ (col & 15)) * 16 : (hh ^ ((col >> 1) & 7)) * 16;
+  auto qk = [&](int kt, f32x16 (&s)[2]) {
+    const uint8_t* kp = lds + (kt & 1) * T_BYTES + col * RB;
 #pragma unroll
-      for (int p = 0; p < KPASS; ++p)
-        kreg[p] = *reinterpret_cast<const u32x4*>(kb + p * KRPP * a.k_tok_b + koff);
-    } else {  // last tile: rows clamped to the sequence (masked in S)
+    for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-      for (int p = 0; p < KPASS; ++p) {
-        const int row = min(r0 + kr + KRPP * p, len - 1);
-        kreg[p] = *reinterpret_cast<const u32x4*>(kbase + row * a.k_tok_b + kc * 16);
-      }
-    }
+      for (int i = 0; i < 16; ++i) s[sb][i] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < W::KS; ++ks)
+#pragma unroll
+      for (int sb = 0; sb < 2; ++sb)
+        s[sb] = E::mfma(*reinterpret_cast<const u32x4*>(kp + (kx ^ (32 * ks)) + 32 * sb * RB),
+                        st.qv[ks], s[sb]);
   };
-  auto load_v = [&](int kt) {
-    if (t >= VTHREADS) return;
-    const int r0 = kt * kPfKTile;
-    if (r0 + kPfKTile <= len) {
-      const uint8_t* vb = vbase + r0 * a.v_tok_b;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        vreg[i] = *reinterpret_cast<const u32x4*>(vb + i * a.v_tok_b + voff);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int row = min(r0 + 4 * vq + i, len - 1);
-        vreg[i] = *reinterpret_cast<const u32x4*>(vbase + row * a.v_tok_b + vc * 16);
-      }
-    }
-  };
-  auto store_k = [&](int slot) {
-    uint8_t* sk = lds + slot * K_BYTES;
-#pragma unroll
-    for (int p = 0; p < KPASS; ++p)
-      *reinterpret_cast<u32x4*>(sk + (kr + KRPP * p) * KPITCH + kc * 16) = kreg[p];
-  };
-  auto store_v = [&](int kt, int slot) {
-    if (t >= VTHREADS) return;
-    if (kt * kPfKTile + kPfKTile > len) {  // last tile only (uniform)
-#pragma unroll
-      for (int i = 0; i < 4; ++i)  // keys past the end: 0 (P is 0 there, V may be NaN)
-        if (kt * kPfKTile + 4 * vq + i >= len) vreg[i] = u32x4{0, 0, 0, 0};
-    }
-    const u32x4* x = vreg;
-    uint8_t* vt = lds + 2 * K_BYTES + slot * V_BYTES + vpos * 2;
-#pragma unroll
-    for (int wd = 0; wd < 4; ++wd) {  // dims 2 wd (low halves) and 2 wd + 1 (high)
-      *reinterpret_cast<u32x2*>(vt + (8 * vc + 2 * wd) * kVtPitch) =
-          u32x2{pack_lo(x[0][wd], x[1][wd]), pack_lo(x[2][wd], x[3][wd])};
-      *reinterpret_cast<u32x2*>(vt + (8 * vc + 2 * wd + 1) * kVtPitch) =
-          u32x2{pack_hi(x[0][wd], x[1][wd]), pack_hi(x[2][wd], x[3][wd])};
-    }
-  };
-  auto pv = [&](int kt, const u32x4 (&pb)[4]) {
-    const uint8_t* vp = lds + 2 * K_BYTES + (kt & 1) * V_BYTES + col * kVtPitch + 16 * hh;
+  // V operand (see the long kernel's transposing reads): lane (G, s) reads 4
+  // dims 32 db + 16 (G & 1) + 4 (s % 4) .. + 3 of key 4 (G >> 1) + s / 4
+  // (+ 16 kk, + 8), whose chunk's bit 2 (and 3) are permuted
+  const int vG = lane >> 4, vs = lane & 15;
+  const int vkey = 4 * (vG >> 1) + (vs >> 2);
+  const int vx = 64 * (D == 128 ? vkey & 3 : (vkey >> 1) & 1);
+  const uint8_t* vp =
+      lds + 2 * T_BYTES + vkey * RB + (2 * (vG & 1) + ((vs & 3) >> 1)) * 16 + 8 * (vs & 1);
+  auto pv = [&](const u32x4 (&pb)[4]) {
 #pragma unroll
     for (int kk = 0; kk < 4; ++kk)
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
-        st.o[db] = E::mfma(*reinterpret_cast<const u32x4*>(vp + 32 * db * kVtPitch + 32 * kk),
-                           pb[kk], st.o[db]);
+      for (int db = 0; db < DB; ++db) {
+        const uint8_t* x = vp + (vx ^ (64 * db)) + 16 * kk * RB;
+        const u32x2 lo = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)x));
+        const u32x2 hi = __builtin_bit_cast(
+            u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(x + 8 * RB)));
+        st.o[db] = E::mfma(u32x4{lo[0], lo[1], hi[0], hi[1]}, pb[kk], st.o[db]);
+      }
+  };
+  auto mine = [&](int kt) {  // the wave has queries that need tile kt (uniform)
+    return wq0 < len && (!a.causal || kt * kPfKTile <= wq0 + kUnitQ - 1);
   };
 
-  // K and V of tile kt + 1 are loaded while tile kt is computed; two
-  // workgroups per CU overlap each other's softmax and matrix work.
-  load_k(0);
-  load_v(0);
-  store_k(0);
-  store_v(0, 0);
-  __syncthreads();
+  // Tile kt: K_{kt+1} and V_kt are loaded while S_kt and its softmax are
+  // computed; they are waited for before the barrier that starts P.V.  V_kt's
+  // stage is free once every wave is past the P.V of tile kt - 1 (the barrier at
+  // the top), K_{kt+1}'s since the S of tile kt - 1.
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // K_0, V_0 and the queries
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
   for (int kt = 0; kt < n_kt; ++kt) {
-    const bool more = kt + 1 < n_kt;
-    if (more) {
-      load_k(kt + 1);
-      load_v(kt + 1);
+    if (kt > 0) {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's V reads
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      dma_v(kt);
     }
-    if (wq0 < len && (!a.causal || kt * kPfKTile <= wq0 + 31)) {
+    if (kt + 1 < n_kt) dma_k(kt + 1);
+    u32x4 pb[4];
+    if (mine(kt)) {
       f32x16 sc[2];
-      u32x4 pb[4];
-      st.template qk<KPITCH, 0>(lds + (kt & 1) * K_BYTES + col * KPITCH + 16 * hh, sc);
+      qk(kt, sc);
       st.mask(sc, kt * kPfKTile, wq0, qi, len, a.causal, hh);
       st.softmax(sc, pb, a.scale_log2);
-      pv(kt, pb);
     }
-    if (more) {
-      store_k((kt + 1) & 1);
-      store_v(kt + 1, (kt + 1) & 1);
-    }
-    __syncthreads();
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (mine(kt)) pv(pb);
   }
   st.store(a, h, s0, len, qi, hh);
 }
 
 template <int DT, int D>
-__global__ __launch_bounds__(kShortThreads, 2) void prefill_short_kernel(PrefillArgs a) {
-  constexpr int K_BYTES = kPfKTile * (D * 2 + 16);
-  constexpr int V_BYTES = D * kVtPitch;
-  // two K stages, then two V^T stages
-  __shared__ __align__(16) uint8_t lds[2 * K_BYTES + 2 * V_BYTES];
+__global__ __launch_bounds__(kShortThreads, 3) void prefill_short_kernel(PrefillArgs a) {
+  // two K stages, then one V stage
+  __shared__ __align__(16) uint8_t lds[3 * kPfKTile * D * 2];
   int kvh, s0, len, u0;
   if (!pick_job<kShortWaves>(a, kvh, s0, len, u0)) return;  // uniform, before any barrier
   attend_short<DT, D>(a, lds, kvh, s0, len, u0);
