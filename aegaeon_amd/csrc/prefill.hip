@@ -266,22 +266,38 @@ struct WaveState {
     }
   }
 
-  // normalise and store the lane's outputs (queries past the end: none)
-  __device__ __forceinline__ void store(const PrefillArgs& a, int h, int64_t s0, int len, int qi,
-                                        int hh) {
+  // normalise and store the wave's outputs (queries past the end: none).  A
+  // lane holds 8-byte pieces of one row, so they go through LDS at `x` (the
+  // wave's own 32 rows of D, 16-byte chunk c of row r at c ^ r % chunks, which
+  // keeps both sides off each other's banks) and leave as whole rows.  (Straight from the
+  // registers, 32 rows x 16 bytes per store, a wave's stores took 2.2 us of a
+  // 20 us job: 48 prompts of 25-766 tokens 82.0 us, so 70.1; 4 x 2048 141.7
+  // and 131.3; 1 x 8192 452 and 435.)
+  __device__ __forceinline__ void store(const PrefillArgs& a, uint8_t* x, int h, int64_t s0,
+                                        int len, int wq0) {
+    constexpr int RB = D * 2, CPR = D / 8, RPI = 64 / CPR;  // bytes, chunks per row; rows per store
+    const int lane = threadIdx.x & 63, col = lane & 31, hh = lane >> 5;
     const float lt = lsum + __shfl_xor(lsum, 32);
-    if (qi < len) {
-      const float inv = 1.f / lt;
-      uint8_t* op = a.out + (s0 + qi) * a.o_tok_b + ((int64_t)h * D + 4 * hh) * 2;
+    const float inv = 1.f / lt;
+    uint8_t* xw = x + col * RB + 8 * hh;
 #pragma unroll
-      for (int db = 0; db < DB; ++db)
+    for (int db = 0; db < DB; ++db)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const f32x16& r = o[db];
-          *reinterpret_cast<u32x2*>(op + (32 * db + 8 * g) * 2) =
-              u32x2{PfOps<DT>::pack(r[4 * g] * inv, r[4 * g + 1] * inv),
-                    PfOps<DT>::pack(r[4 * g + 2] * inv, r[4 * g + 3] * inv)};
-        }
+      for (int g = 0; g < 4; ++g) {
+        const f32x16& r = o[db];
+        *reinterpret_cast<u32x2*>(xw + ((4 * db + g) ^ (col % CPR)) * 16) =
+            u32x2{PfOps<DT>::pack(r[4 * g] * inv, r[4 * g + 1] * inv),
+                  PfOps<DT>::pack(r[4 * g + 2] * inv, r[4 * g + 3] * inv)};
+      }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // the wave's own writes
+    const int row = lane / CPR, pos = lane % CPR;
+    uint8_t* op = a.out + (s0 + wq0) * a.o_tok_b + (int64_t)h * RB;
+#pragma unroll
+    for (int i = 0; i < 32 / RPI; ++i) {
+      const int r = RPI * i + row;
+      const u32x4 v = *reinterpret_cast<const u32x4*>(x + 1024 * i + 16 * lane);
+      if (wq0 + r < len)
+        *reinterpret_cast<u32x4*>(op + r * a.o_tok_b + (pos ^ (r % CPR)) * 16) = v;
     }
   }
 };
@@ -499,7 +515,8 @@ __device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds,
     asm volatile("" ::: "memory");
     if (mine(kt)) pv(pb);
   }
-  st.store(a, h, s0, len, qi, hh);
+  // the K stages: every wave is past its last read of them
+  st.store(a, lds + w * (kUnitQ * RB), h, s0, len, wq0);
 }
 
 template <int DT, int D>
@@ -676,7 +693,10 @@ __device__ __forceinline__ void attend_long(const PrefillArgs& a, uint8_t* lds, 
     }
     if (n_kt - 1 <= jw) pv(n_kt - 1, pb);  // slot 2 n_kt
     PF_BARRIER();
-    PF_BARRIER();  // slot 2 n_kt + 1: idle
+    // slot 2 n_kt + 1: the outputs, through the K stages (last read in slot
+    // 2 n_kt - 1), while the other half runs its last P.V
+    st.store(a, lds + w * (kUnitQ * D * 2), h, s0, len, wq0);
+    PF_BARRIER();
   } else {
     stage(0);  // slot 0: idle
     PF_BARRIER();
@@ -691,10 +711,11 @@ __device__ __forceinline__ void attend_long(const PrefillArgs& a, uint8_t* lds, 
     }
     if (n_kt - 1 <= jw) pv(n_kt - 1, pb);  // slot 2 n_kt + 1
     PF_BARRIER();
+    // through the V stages, whose last reads were this half's
+    st.store(a, lds + 2 * K_BYTES + (w - 4) * (kUnitQ * D * 2), h, s0, len, wq0);
   }
 #undef PF_BARRIER
 #undef PF_BARRIER_LOADED
-  st.store(a, h, s0, len, qi, hh);
 }
 
 template <int DT, int D>

@@ -314,3 +314,22 @@ def test_jobs_over_existing_tiles(Hq, Hkv, top, causal):
     assert torch.equal(first.view(torch.int16), all_[:n].view(torch.int16))
     assert torch.equal(few.view(torch.int16), all_[:int(cu[8])].view(torch.int16))
     _check(few, q, k, v, cu[:9], 0.125, causal, torch.bfloat16, int(cu[8]))
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("top", [95, 1601])  # the four-wave and the ping-pong kernel
+def test_output_rows_leave_whole(D, top):
+    """The outputs pass through LDS and are stored as rows: prompts that end on
+    every side of a 32-query unit, into a slice of a wider buffer whose other
+    rows and columns keep their bytes."""
+    Hq, Hkv, pad = 6, 2, 24
+    lens = [1, 31, 32, 33, 63, 64, 65, top]
+    cu, q, k, v = _packed(lens, Hq, Hkv, D, torch.bfloat16, 29, extra=2)
+    T = q.size(0)
+    wide = torch.full((T, Hq * D + 2 * pad), 7.0, dtype=q.dtype, device="cuda")
+    out = wide[:, pad:pad + Hq * D].unflatten(1, (Hq, D))
+    A.varlen_prefill_attention(q, k, v, torch.from_numpy(cu).cuda(), top, 0.1, True, out=out)
+    _check(out, q, k, v, cu, 0.1, True, torch.bfloat16)
+    n = int(cu[-1])
+    assert (wide[:, :pad] == 7.0).all() and (wide[:, pad + Hq * D:] == 7.0).all()
+    assert (wide[n:] == 7.0).all()
