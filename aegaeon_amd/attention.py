@@ -23,20 +23,18 @@ from typing import Dict, Optional, Sequence, Tuple
 import torch
 
 from . import _lib
+from ._gpu import device_guard, raw_stream
 
 _DTYPES = {torch.bfloat16: _lib.AEGKV_DTYPE_BF16, torch.float16: _lib.AEGKV_DTYPE_FP16}
-
-
-def _stream(t: torch.Tensor) -> int:
-    return torch.cuda.current_stream(t.device).cuda_stream
 
 
 def _check_cache_view(c: torch.Tensor, name: str) -> None:
     """A per-layer cache view ``[N, bs, Hkv, D]`` with dense rows per block."""
     if c.dim() != 4 or not c.is_cuda:
         raise ValueError(f"{name} must be a 4-d GPU tensor [N, block_size, Hkv, D]")
-    N, bs, H, D = c.shape
-    if c.stride(3) != 1 or c.stride(2) != D or c.stride(1) != H * D:
+    _, _, H, D = c.shape
+    strides = c.stride()
+    if strides[3] != 1 or strides[2] != D or strides[1] != H * D:
         raise ValueError(f"{name}: each block must hold dense [block_size, Hkv, D] rows")
 
 
@@ -47,7 +45,8 @@ def _check_on(t: torch.Tensor, name: str, device: torch.device) -> None:
 
 
 def _check_rows(x: torch.Tensor, name: str) -> None:
-    if not x.is_cuda or x.stride(-1) != 1 or x.stride(-2) != x.size(-1):
+    strides = x.stride()
+    if not x.is_cuda or strides[-1] != 1 or strides[-2] != x.size(-1):
         raise ValueError(f"{name}: rows [Hkv, D] must be dense on the GPU")
 
 
@@ -85,11 +84,12 @@ def reshape_and_cache_flash(key: torch.Tensor, value: torch.Tensor, key_cache: t
         raise ValueError(f"slot_mapping must hold a slot for each of the {T} tokens")
     N, bs, H, D = key_cache.shape
     slot_mapping = slot_mapping.contiguous()
-    with torch.cuda.device(key.device):
+    dev = key_cache.device
+    with device_guard(dev):
         rc = _lib.load().aegkv_kv_append(
             key.data_ptr(), value.data_ptr(), key.stride(0), value.stride(0), 0, 0,
             slot_mapping.data_ptr(), T, key_cache.data_ptr(), value_cache.data_ptr(),
-            key_cache.stride(0), 0, N, 1, bs, H, D, key.element_size(), _stream(key))
+            key_cache.stride(0), 0, N, 1, bs, H, D, 2, raw_stream(dev))
     _lib.check(rc, "reshape_and_cache_flash")
 
 
@@ -117,14 +117,14 @@ def append_kv(key: torch.Tensor, value: torch.Tensor, kv_cache: torch.Tensor,
     if slot_mapping.dim() != 1 or slot_mapping.numel() < T:
         raise ValueError(f"slot_mapping must hold a slot for each of the {T} tokens")
     slot_mapping = slot_mapping.contiguous()
-    kv_stride = bs * H * D
-    with torch.cuda.device(kv_cache.device):
+    dev = kv_cache.device
+    ks, vs, cs = key.stride(), value.stride(), kv_cache.stride()
+    with device_guard(dev):
         base = kv_cache.data_ptr()
         rc = _lib.load().aegkv_kv_append(
-            key.data_ptr(), value.data_ptr(), key.stride(1), value.stride(1), key.stride(0),
-            value.stride(0), slot_mapping.data_ptr(), T, base,
-            base + kv_stride * kv_cache.element_size(), kv_cache.stride(0), kv_cache.stride(1), N,
-            L, bs, H, D, kv_cache.element_size(), _stream(kv_cache))
+            key.data_ptr(), value.data_ptr(), ks[1], vs[1], ks[0], vs[0],
+            slot_mapping.data_ptr(), T, base, base + 2 * bs * H * D, cs[0], cs[1], N, L, bs, H, D,
+            2, raw_stream(dev))
     _lib.check(rc, "append_kv")
 
 
@@ -166,13 +166,13 @@ def gather_tokens(kv_cache: torch.Tensor, block_tables: torch.Tensor, seq_lens: 
     if total_tokens == 0:
         return out_k, out_v
     es = kv_cache.element_size()
-    with torch.cuda.device(kv_cache.device):
+    with device_guard(kv_cache.device):
         base = kv_cache.data_ptr() + first * kv_cache.stride(1) * es
         rc = _lib.load().aegkv_gather_tokens(
             base, base + bs * H * D * es, kv_cache.stride(0), kv_cache.stride(1), N,
             bt.data_ptr(), bt.size(1), sl.data_ptr(), cu_seqlens.data_ptr(), sl.numel(),
             max_seq_len, out_k.data_ptr(), out_v.data_ptr(), total_tokens, total_tokens * H * D,
-            count, bs, H, D, es, _stream(kv_cache))
+            count, bs, H, D, es, raw_stream(kv_cache.device))
     _lib.check(rc, "gather_tokens")
     return out_k, out_v
 
@@ -195,7 +195,7 @@ def attention_workspace_bytes(batch: int, n_q_heads: int, n_kv_heads: int, head_
     if dtype not in _DTYPES:
         raise ValueError("dtype must be bfloat16 or float16")
     dev = _gpu(device)
-    with torch.cuda.device(dev):
+    with device_guard(dev):
         n = _lib.load().aegkv_paged_decode_attention_workspace_size(
             batch, n_q_heads, n_kv_heads, head_dim, max_seq_len, _DTYPES[dtype], n_workgroups)
     if n < 0:
@@ -260,7 +260,7 @@ class DecodePlan:
         self.n_workgroups = int(n_workgroups)
         dev = self.seq_lens.device
         lib = _lib.load()
-        with torch.cuda.device(dev):
+        with device_guard(dev):
             n = lib.aegkv_paged_decode_plan_size(self.batch, self.n_kv_heads, self.max_seq_len,
                                                   self.n_workgroups)
             if n < 0:
@@ -268,10 +268,11 @@ class DecodePlan:
             self.buffer = torch.empty(max(int(n), 1), dtype=torch.uint8, device=dev)
             self.nbytes = int(n)
             stream = torch.cuda.current_stream(dev)
+            self.raw_stream = stream.cuda_stream
             rc = lib.aegkv_paged_decode_plan(
                 self.block_tables.data_ptr(), self.block_tables.size(1), self.seq_lens.data_ptr(),
                 self.batch, self.max_seq_len, self.n_kv_heads, self.n_workgroups,
-                self.buffer.data_ptr(), self.nbytes, stream.cuda_stream)
+                self.buffer.data_ptr(), self.nbytes, self.raw_stream)
             _lib.check(rc, "decode_plan")
             # Calls on another stream wait for the build (wait_for_build).
             self.stream = stream
@@ -343,10 +344,9 @@ def paged_decode_attention(q: torch.Tensor, key_cache: torch.Tensor, value_cache
         raise ValueError("q, key_cache and value_cache must share a bf16/fp16 dtype")
     B, Hq, D = q.shape
     N, bs, Hkv, _ = key_cache.shape
-    bt = _int32_dense(block_tables)
     sl = _int32_dense(seq_lens)
     if out is None:
-        out = torch.empty((B, Hq, D), dtype=q.dtype, device=q.device)
+        out = torch.empty((B, Hq, D), dtype=q.dtype, device=dev)
     elif out.shape != (B, Hq, D) or out.stride(2) != 1 or out.stride(1) != D:
         raise ValueError("out must be [B, Hq, D] with dense heads")
     elif out.dtype != q.dtype:
@@ -355,17 +355,6 @@ def paged_decode_attention(q: torch.Tensor, key_cache: torch.Tensor, value_cache
         _check_on(out, "out", dev)
     if B == 0:
         return out
-    ws_bytes = attention_workspace_bytes(B, Hq, Hkv, D, max_seq_len, q.dtype, n_workgroups,
-                                         q.device)
-    if ws_bytes > 0 and workspace is None:
-        workspace = _cached_workspace(q.device, _stream(q), ws_bytes)
-    if ws_bytes > 0:
-        _check_on(workspace, "workspace", dev)
-        if workspace.numel() * workspace.element_size() < ws_bytes:
-            raise ValueError(f"workspace holds {workspace.numel() * workspace.element_size()} "
-                             f"bytes, the call needs {ws_bytes}")
-    if plan is not None:
-        plan.wait_for_build(torch.cuda.current_stream(dev))
     if (key is None) != (value is None):
         raise ValueError("key and value are appended together")
     if key is not None:
@@ -374,36 +363,40 @@ def paged_decode_attention(q: torch.Tensor, key_cache: torch.Tensor, value_cache
                 raise ValueError(f"{n} must be [B, Hkv, D] of q's dtype")
             _check_rows(t, n)
             _check_on(t, n, dev)
-    ws_ptr = workspace.data_ptr() if (workspace is not None and ws_bytes > 0) else None
-    with torch.cuda.device(q.device):
+    lib = _lib.load()
+    dtype = _DTYPES[q.dtype]
+    with device_guard(dev):
+        ws_bytes = lib.aegkv_paged_decode_attention_workspace_size(B, Hq, Hkv, D, max_seq_len,
+                                                                   dtype, n_workgroups)
+        if ws_bytes < 0:
+            _lib.check(int(ws_bytes), "attention_workspace_bytes")
+        stream = raw_stream(dev)
+        ws_ptr = None
+        if ws_bytes > 0:
+            if workspace is None:
+                workspace = _cached_workspace(dev, stream, ws_bytes)
+            _check_on(workspace, "workspace", dev)
+            if workspace.numel() * workspace.element_size() < ws_bytes:
+                raise ValueError(f"workspace holds {workspace.numel() * workspace.element_size()} "
+                                 f"bytes, the call needs {ws_bytes}")
+            ws_ptr = workspace.data_ptr()
+        if plan is not None and stream != plan.raw_stream:
+            plan.wait_for_build(torch.cuda.current_stream(dev))
+        args = (out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0))
         if key is not None:
-            kv = (key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0))
-            if plan is not None:
-                rc = _lib.load().aegkv_paged_decode_attention_append_planned(
-                    out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), *kv,
-                    key_cache.data_ptr(), value_cache.data_ptr(), key_cache.stride(0), N,
-                    plan.buffer.data_ptr(), plan.nbytes, sl.data_ptr(), B, max_seq_len, Hq, Hkv,
-                    D, bs, float(scale), _DTYPES[q.dtype], n_workgroups, ws_ptr,
-                    ws_bytes if ws_ptr else 0, _stream(q))
-            else:
-                rc = _lib.load().aegkv_paged_decode_attention_append(
-                    out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), *kv,
-                    key_cache.data_ptr(), value_cache.data_ptr(), key_cache.stride(0), N,
-                    bt.data_ptr(), bt.size(1), sl.data_ptr(), B, max_seq_len, Hq, Hkv, D, bs,
-                    float(scale), _DTYPES[q.dtype], n_workgroups, ws_ptr,
-                    ws_bytes if ws_ptr else 0, _stream(q))
-        elif plan is not None:
-            rc = _lib.load().aegkv_paged_decode_attention_planned(
-                out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), key_cache.data_ptr(),
-                value_cache.data_ptr(), key_cache.stride(0), N, plan.buffer.data_ptr(),
-                plan.nbytes, sl.data_ptr(), B, max_seq_len, Hq, Hkv, D, bs, float(scale),
-                _DTYPES[q.dtype], n_workgroups, ws_ptr, ws_bytes if ws_ptr else 0, _stream(q))
+            args += (key.data_ptr(), key.stride(0), value.data_ptr(), value.stride(0))
+        args += (key_cache.data_ptr(), value_cache.data_ptr(), key_cache.stride(0), N)
+        if plan is not None:
+            args += (plan.buffer.data_ptr(), plan.nbytes)
+            call = lib.aegkv_paged_decode_attention_planned if key is None \
+                else lib.aegkv_paged_decode_attention_append_planned
         else:
-            rc = _lib.load().aegkv_paged_decode_attention(
-                out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), key_cache.data_ptr(),
-                value_cache.data_ptr(), key_cache.stride(0), N, bt.data_ptr(), bt.size(1),
-                sl.data_ptr(), B, max_seq_len, Hq, Hkv, D, bs, float(scale), _DTYPES[q.dtype],
-                n_workgroups, ws_ptr, ws_bytes if ws_ptr else 0, _stream(q))
+            bt = _int32_dense(block_tables)
+            args += (bt.data_ptr(), bt.size(1))
+            call = lib.aegkv_paged_decode_attention if key is None \
+                else lib.aegkv_paged_decode_attention_append
+        rc = call(*args, sl.data_ptr(), B, max_seq_len, Hq, Hkv, D, bs, float(scale), dtype,
+                  n_workgroups, ws_ptr, ws_bytes if ws_ptr else 0, stream)
     _lib.check(rc, "paged_decode_attention")
     return out
 
@@ -426,7 +419,7 @@ class _StepPlans:
 
     @staticmethod
     def _state(t: torch.Tensor) -> tuple:
-        return (t._version, t.data_ptr(), tuple(t.shape), tuple(t.stride()), t.dtype)
+        return (t._version, t.data_ptr(), t.shape, t.stride(), t.dtype)
 
     def get(self, block_table: torch.Tensor, cache_seqlens: torch.Tensor, appending: bool,
             max_seq_len: int, n_kv_heads: int):
@@ -530,12 +523,12 @@ def varlen_prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor,
     else:
         _check_rows(out, "out")
         _check_on(out, "out", q.device)
-    with torch.cuda.device(q.device):
+    with device_guard(q.device):
         rc = _lib.load().aegkv_varlen_prefill_attention(
             out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0), k.data_ptr(), k.stride(0),
             v.data_ptr(), v.stride(0), cu_seqlens.data_ptr(), cu_seqlens.numel() - 1,
             int(max_seqlen), T, Hq, k.size(1), D, float(scale), int(bool(causal)),
-            _DTYPES[q.dtype], _stream(q))
+            _DTYPES[q.dtype], raw_stream(q.device))
     _lib.check(rc, "varlen_prefill_attention")
     return out
 

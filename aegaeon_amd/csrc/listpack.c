@@ -14,7 +14,15 @@
  *       does not hold seq_len - context_len tokens raises ValueError
  *
  * Both accept lists or tuples (any sequence) of Python ints and raise
- * TypeError / OverflowError for anything else. */
+ * TypeError / OverflowError for anything else.
+ *
+ *   step_counts(offsets, seq_lens, context_lens) ->
+ *       (seq_lens as a list, new tokens, longest decode table, prefills,
+ *        prefill tokens, longest new part, longest prefill, longest decode)
+ *       of such buffers (requests of context 0 are prefills; a maximum over
+ *       none is 0): the step's counts that the host keeps, in one pass
+ *   address(buffer) -> its address as an int (None when empty); the caller
+ *       keeps the buffer alive while it uses the address */
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -159,11 +167,79 @@ fail:
   return NULL;
 }
 
+static PyObject* step_counts(PyObject* self, PyObject* args) {
+  (void)self;
+  Py_buffer off, seq, ctx;
+  if (!PyArg_ParseTuple(args, "y*y*y*", &off, &seq, &ctx)) return NULL;
+  PyObject* list = NULL;
+  PyObject* out = NULL;
+  const Py_ssize_t n = seq.len / (Py_ssize_t)sizeof(int32_t);
+  if (n == 0 || ctx.len != seq.len || off.len != (n + 1) * (Py_ssize_t)sizeof(int64_t)) {
+    PyErr_SetString(PyExc_ValueError, "one context length and one table per request");
+    goto done;
+  }
+  list = PyList_New(n);
+  if (!list) goto done;
+  const int64_t* o = (const int64_t*)off.buf;
+  const int32_t* s = (const int32_t*)seq.buf;
+  const int32_t* c = (const int32_t*)ctx.buf;
+  /* unsigned sums: any lengths, also ones the call then refuses */
+  uint64_t total = 0, prompt_total = 0;
+  int64_t prompts = 0, longest_new = INT64_MIN;
+  int64_t width = INT64_MIN, longest_prompt = INT64_MIN, longest_decode = INT64_MIN;
+  for (Py_ssize_t b = 0; b < n; ++b) {
+    const int64_t fresh = (int64_t)s[b] - c[b];
+    PyObject* v = PyLong_FromLong(s[b]);
+    if (!v) goto done;
+    PyList_SET_ITEM(list, b, v);
+    total += (uint64_t)fresh;
+    if (fresh > longest_new) longest_new = fresh;
+    if (c[b] == 0) {
+      ++prompts;
+      prompt_total += (uint64_t)fresh;
+      if (s[b] > longest_prompt) longest_prompt = s[b];
+    } else {
+      const int64_t w = (int64_t)((uint64_t)o[b + 1] - (uint64_t)o[b]);
+      if (w > width) width = w;
+      if (s[b] > longest_decode) longest_decode = s[b];
+    }
+  }
+  if (prompts == n) width = longest_decode = 0;
+  if (prompts == 0) longest_prompt = 0;
+  out = Py_BuildValue("(OLLLLLLL)", list, (long long)total, (long long)width, (long long)prompts,
+                      (long long)prompt_total, (long long)longest_new, (long long)longest_prompt,
+                      (long long)longest_decode);
+done:
+  Py_XDECREF(list);
+  PyBuffer_Release(&off);
+  PyBuffer_Release(&seq);
+  PyBuffer_Release(&ctx);
+  return out;
+}
+
+static PyObject* address(PyObject* self, PyObject* arg) {
+  (void)self;
+  Py_buffer b;
+  if (PyObject_GetBuffer(arg, &b, PyBUF_SIMPLE)) return NULL;
+  PyObject* out;
+  if (b.len == 0) {
+    out = Py_None;
+    Py_INCREF(out);
+  } else {
+    out = PyLong_FromVoidPtr(b.buf);
+  }
+  PyBuffer_Release(&b);
+  return out;
+}
+
 static PyMethodDef methods[] = {
     {"pack_tables", pack_tables, METH_O,
      "pack_tables(tables) -> (int32 ids bytearray, int64 offsets bytearray)"},
     {"pack_requests", pack_requests, METH_O,
      "pack_requests(requests) -> (int32 seq_lens, int32 context_lens, int64 tokens) bytearrays"},
+    {"step_counts", step_counts, METH_VARARGS,
+     "step_counts(offsets, seq_lens, context_lens) -> (list, seven counts)"},
+    {"address", address, METH_O, "address(buffer) -> int, None when it is empty"},
     {NULL, NULL, 0, NULL}};
 
 static struct PyModuleDef module = {PyModuleDef_HEAD_INIT, "_listpack",

@@ -19,6 +19,7 @@ import numpy as np
 import torch
 
 from . import _lib
+from ._gpu import device_guard, raw_stream
 
 try:
     from . import _listpack
@@ -27,10 +28,6 @@ except ImportError as e:  # built beside libaegkv.so by csrc/build.py
                       "(aegaeon_amd/csrc/build.py)") from e
 
 BLOCK_SIZE = 16  # aegaeon/aegaeon/config.py:13
-
-
-def _ptr(a: np.ndarray):
-    return a.ctypes.data if a.size else None
 
 
 def prepare_model_inputs(requests: Sequence[Tuple], block_tables: Sequence[Sequence[int]],
@@ -55,11 +52,7 @@ def prepare_model_inputs(requests: Sequence[Tuple], block_tables: Sequence[Seque
     # manager's tables, the requests' lengths and new tokens)
     ids, offsets = _listpack.pack_tables(block_tables)
     seq, ctx, tokens = _listpack.pack_requests(requests)
-    return prepare_inputs_from_arrays(np.frombuffer(ids, dtype=np.int32),
-                                      np.frombuffer(offsets, dtype=np.int64),
-                                      np.frombuffer(seq, dtype=np.int32),
-                                      np.frombuffer(ctx, dtype=np.int32),
-                                      np.frombuffer(tokens, dtype=np.int64), device, block_size)
+    return _prepare(ids, offsets, seq, ctx, tokens, len(tokens) // 8, device, block_size)
 
 
 def prepare_inputs_from_arrays(table_ids: np.ndarray, table_offsets: np.ndarray,
@@ -71,7 +64,6 @@ def prepare_inputs_from_arrays(table_ids: np.ndarray, table_offsets: np.ndarray,
     (int32; the layout ``BlockManager.flat_block_tables`` returns), its
     lengths ``seq_lens[b]`` / ``context_lens[b]`` (int32) and its new tokens
     the next ``seq_len - context_len`` entries of ``tokens`` (int64)."""
-    device = torch.device(device)
     ids = np.ascontiguousarray(table_ids, dtype=np.int32)
     offsets = np.ascontiguousarray(table_offsets, dtype=np.int64)
     seq = np.ascontiguousarray(seq_lens, dtype=np.int32)
@@ -82,42 +74,50 @@ def prepare_inputs_from_arrays(table_ids: np.ndarray, table_offsets: np.ndarray,
         raise ValueError("empty batch")  # the reference asserts (worker.py:594)
     if ctx.size != B or offsets.size != B + 1:
         raise ValueError("one context length and one table per request")
-    qlen = seq.astype(np.int64) - ctx
-    is_prompt = ctx == 0
-    lens = np.diff(offsets)
-    # decode rows keep their table, prefill rows are empty (worker.py:600-605)
-    pad_width = int(lens[~is_prompt].max()) if (~is_prompt).any() else 0
-    T = int(qlen.sum())
-    if tokens.size != T:
+    return _prepare(ids, offsets, seq, ctx, tokens, tokens.size, device, block_size)
+
+
+def _prepare(ids, offsets, seq, ctx, tokens, n_tokens: int, device, block_size: int
+             ) -> Tuple[torch.Tensor, torch.Tensor, Dict]:
+    """The step's outputs from host buffers (int32 ids, int64 offsets, int32
+    lengths, int64 tokens)."""
+    device = torch.device(device)
+    # decode rows keep their table, prefill rows are empty (worker.py:600-605):
+    # pad_width is the longest table of a decode row
+    (seq_list, T, pad_width, num_prefills, prefill_tokens, max_query, max_prefill,
+     max_decode) = _listpack.step_counts(offsets, seq, ctx)
+    if n_tokens != T:
         raise ValueError("tokens must hold every request's new tokens")
+    B = len(seq_list)
 
     # the outputs are views of one int32 and one int64 allocation (two
     # allocator calls per step instead of eight)
     w32 = torch.empty(B * pad_width + 4 * B + 2, dtype=torch.int32, device=device)
     w64 = torch.empty(3 * T, dtype=torch.int64, device=device)
-    bt_out = w32[:B * pad_width].view(B, pad_width)
-    seq_t, ctx_t, qsl, ssl = torch.split(w32[B * pad_width:], [B, B, B + 1, B + 1])
-    slots, positions, toks = torch.split(w64, [T, T, T])
-    with torch.cuda.device(device):
+    bt_out, seq_t, ctx_t, qsl, ssl = w32.split_with_sizes([B * pad_width, B, B, B + 1, B + 1])
+    bt_out = bt_out.view(B, pad_width)
+    slots, positions, toks = w64.split_with_sizes([T, T, T])
+    p32 = w32.data_ptr()
+    p_seq = p32 + 4 * B * pad_width
+    p64 = w64.data_ptr()
+    address = _listpack.address
+    with device_guard(device):
         rc = _lib.load().aegkv_prepare_inputs(
-            _ptr(ids), offsets.ctypes.data, seq.ctypes.data, ctx.ctypes.data, _ptr(tokens), B,
-            block_size, pad_width, bt_out.data_ptr() if pad_width else None,
-            slots.data_ptr() if T else None, positions.data_ptr() if T else None,
-            toks.data_ptr() if T else None, seq_t.data_ptr(), ctx_t.data_ptr(), qsl.data_ptr(),
-            ssl.data_ptr(), T, torch.cuda.current_stream(device).cuda_stream)
+            address(ids), address(offsets), address(seq), address(ctx), address(tokens), B,
+            block_size, pad_width, p32 if pad_width else None, p64 if T else None,
+            p64 + 8 * T if T else None, p64 + 16 * T if T else None, p_seq, p_seq + 4 * B,
+            p_seq + 8 * B, p_seq + 12 * B + 4, T, raw_stream(device))
     _lib.check(rc, "prepare_model_inputs")
-    prefill_lens = seq[is_prompt]
-    decode_lens = seq[~is_prompt]
     metadata = dict(
-        num_prefills=int(is_prompt.sum()),
+        num_prefills=num_prefills,
         slot_mapping=slots,
-        num_prefill_tokens=int(qlen[is_prompt].sum()),
-        num_decode_tokens=int(qlen[~is_prompt].sum()),
-        seq_lens=seq.tolist(),
+        num_prefill_tokens=prefill_tokens,
+        num_decode_tokens=T - prefill_tokens,
+        seq_lens=seq_list,
         seq_lens_tensor=seq_t,
-        max_query_len=int(qlen.max()),
-        max_prefill_seq_len=int(prefill_lens.max()) if prefill_lens.size else 0,
-        max_decode_seq_len=int(decode_lens.max()) if decode_lens.size else 0,
+        max_query_len=max_query,
+        max_prefill_seq_len=max_prefill,
+        max_decode_seq_len=max_decode,
         query_start_loc=qsl,
         seq_start_loc=ssl,
         context_lens_tensor=ctx_t,

@@ -46,3 +46,39 @@ def test_errors():
         _listpack.pack_tables([[2 ** 31]])
     with pytest.raises(OverflowError):
         _listpack.pack_requests([(0, [], 2 ** 31, 2 ** 31)])
+
+
+def _counts(offsets, seq, ctx):
+    """step_counts by numpy over int64."""
+    qlen = seq.astype(np.int64) - ctx
+    prompt = ctx == 0
+    top = lambda x: int(x.max()) if x.size else 0
+    return (seq.tolist(), int(qlen.sum()), top(np.diff(offsets)[~prompt]), int(prompt.sum()),
+            int(qlen[prompt].sum()), int(qlen.max()), top(seq[prompt]), top(seq[~prompt]))
+
+
+@pytest.mark.parametrize("n,prompts", [(1, 0.0), (1, 1.0), (7, 0.5), (300, 0.0), (300, 1.0),
+                                       (513, 0.3)])
+def test_step_counts_like_numpy(n, prompts):
+    rng = np.random.default_rng(n)
+    ctx = rng.integers(1, 5000, n).astype(np.int32)
+    ctx[rng.random(n) < prompts] = 0
+    seq = (ctx + rng.integers(0, 400, n)).astype(np.int32)
+    offsets = np.concatenate([[0], np.cumsum(rng.integers(0, 40, n))]).astype(np.int64)
+    want = _counts(offsets, seq, ctx)
+    assert _listpack.step_counts(offsets, seq, ctx) == want
+    assert _listpack.step_counts(bytearray(offsets), bytearray(seq), bytearray(ctx)) == want
+
+
+def test_step_counts_errors_and_address():
+    seq = np.ones(3, dtype=np.int32)
+    with pytest.raises(ValueError):
+        _listpack.step_counts(np.zeros(3, dtype=np.int64), seq, seq)
+    with pytest.raises(ValueError):
+        _listpack.step_counts(np.zeros(4, dtype=np.int64), seq, seq[:2])
+    with pytest.raises(ValueError):
+        _listpack.step_counts(np.zeros(1, dtype=np.int64), seq[:0], seq[:0])
+    assert _listpack.address(seq) == seq.ctypes.data
+    assert _listpack.address(bytearray()) is None
+    with pytest.raises((TypeError, BufferError, ValueError)):
+        _listpack.address(np.ones((4, 4))[:, 1])
