@@ -333,3 +333,19 @@ def test_output_rows_leave_whole(D, top):
     n = int(cu[-1])
     assert (wide[:, :pad] == 7.0).all() and (wide[:, pad + Hq * D:] == 7.0).all()
     assert (wide[n:] == 7.0).all()
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 256, 257])  # a set's and all sets' last and next
+@pytest.mark.parametrize("Hq,Hkv", [(3, 3), (10, 2), (13, 1)])
+def test_job_search_sequence_counts(n, Hq, Hkv):
+    """Ragged prompts on both sides of the sequence counts where the search for
+    a workgroup's job changes, at head counts that are no powers of two; a
+    second run with the bound loosened numbers the same jobs another way."""
+    rng = np.random.default_rng(n)
+    lens = rng.integers(1, 70, n).tolist()
+    lens[-1] = 1
+    cu, q, k, v = _packed(lens, Hq, Hkv, 64, torch.bfloat16, n)
+    cut = torch.from_numpy(cu).cuda()
+    out = A.varlen_prefill_attention(q, k, v, cut, max(lens), 0.1, True)
+    _check(out, q, k, v, cu, 0.1, True, torch.bfloat16)
+    assert torch.equal(out, A.varlen_prefill_attention(q, k, v, cut, max(lens) + 200, 0.1, True))
