@@ -26,7 +26,7 @@
 // host picks one by the batch's longest prompt:
 //
 // Long prompts (max_seqlen > kLongPrompt): ping-pong.  A workgroup of eight
-// waves takes 256 queries of one head and fills a CU; waves w and w + 4 share
+// waves takes eight units of 32 queries and fills a CU; waves w and w + 4 share
 // a SIMD, and the two halves of the workgroup run opposite phases between
 // workgroup barriers.  Per key tile j a wave runs a matrix phase (S_j and the
 // previous tile's O += V_{j-1}^T . P_{j-1}, 32 MFMAs at D = 128) and then a
@@ -38,11 +38,10 @@
 //
 // Short prompts: three workgroups of four waves per CU that overlap each
 // other's latencies, softmax and matrix work unordered; K and V reach LDS the
-// same way.  (With short prompts the ping-pong workgroup's start-up and its larger
-// causal diagonal cost more than the phase overlap gains: 8 x 1024 tokens
-// 112.6 against 109.0 us, 16 x 512 90.1 against 78.5 us; from 2048 tokens on it
-// is faster: 4 x 2048 cache-cold 174.0 against 181.0 us, 2 x 4096 269.5
-// against 303.7 us, 1 x 8192 544.7 against 627.3 us.)
+// same way.  (With short prompts the ping-pong workgroup's start-up costs more
+// than the phase overlap gains, four-wave against ping-pong: 16 x 512 54.4 and
+// 63.9 us, 8 x 1024 78.9 and 83.2; from 2048 tokens on the overlap wins: 4 x
+// 2048 131.6 and 130.1, 2 x 4096 270 and 252, 1 x 8192 464 and 423.)
 //
 // Wave units, both kernels: the work of a (sequence, kv head) pair is cut into
 // units of 32 queries of one query head, unit u = query block u / G of the
@@ -224,24 +223,27 @@ struct WaveState {
 
   // -inf where a key of the tile at k0 is past the end or (causal) after the
   // query; only the tiles that reach past the wave's first query wq0 or the
-  // end need it
+  // end need it.  One comparison with a constant per score: the lane's last key
+  // is counted from its first score's.  (Two comparisons of a key number per
+  // score, and a first tile that rescaled its zero sums: 48 prompts of 25-766
+  // tokens 69.9 us, so 68.8; 4 x 2048 133.2 and 129.0; 1 x 8192 436 and 433.)
   __device__ __forceinline__ void mask(f32x16 (&s)[2], int k0, int wq0, int qi, int len,
                                        int causal, int hh) const {
     if ((causal && k0 + kPfKTile - 1 > wq0) || k0 + kPfKTile > len) {
+      const int last = (causal ? min(qi, len - 1) : len - 1) - k0 - 4 * hh;
 #pragma unroll
       for (int sb = 0; sb < 2; ++sb)
 #pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int kv = k0 + 32 * sb + 8 * (i >> 2) + 4 * hh + (i & 3);
-          const bool ok = kv < len && (!causal || kv <= qi);
-          s[sb][i] = ok ? s[sb][i] : -INFINITY;
-        }
+        for (int i = 0; i < 16; ++i)
+          s[sb][i] = last >= 32 * sb + 8 * (i >> 2) + (i & 3) ? s[sb][i] : -INFINITY;
     }
   }
 
   // online softmax of a masked S^T tile into the P^T operands of its four
   // 16-key steps
-  __device__ __forceinline__ void softmax(f32x16 (&s)[2], u32x4 (&pb)[4], float scale_log2) {
+  // (`first`: the wave's first tile, whose sums are still zero)
+  __device__ __forceinline__ void softmax(f32x16 (&s)[2], u32x4 (&pb)[4], float scale_log2,
+                                          bool first) {
     // raw-score max (the scale is positive) over four chains of triples: a lone
     // pair of scores would be canonicalised first (28 instructions, now 16:
     // 1 x 8192 435.5 -> 427.0 us, 4 x 2048 131.3 -> 128.9)
@@ -267,7 +269,9 @@ struct WaveState {
     const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(bm), __float_as_uint(bm),
                                                      false, false);
     bm = fmaxf(fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1])), bm) * scale_log2;
-    if (__builtin_amdgcn_ballot_w64(bm > m + kPfRescaleSlack)) {
+    if (first) {
+      m = fmaxf(m, bm);
+    } else if (__builtin_amdgcn_ballot_w64(bm > m + kPfRescaleSlack)) {
       const float mn = fmaxf(m, bm);
       const float alpha = __builtin_amdgcn_exp2f(m - mn);  // 0 while m = -inf
       lsum *= alpha;
@@ -554,7 +558,7 @@ __device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds,
       f32x16 sc[2];
       qk(kt, sc);
       st.mask(sc, kt * kPfKTile, wq0, qi, len, a.causal, hh);
-      st.softmax(sc, pb, a.scale_log2);
+      st.softmax(sc, pb, a.scale_log2, kt == 0);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -698,7 +702,7 @@ __device__ __forceinline__ void attend_long(const PrefillArgs& a, uint8_t* lds, 
   };
   auto softmax = [&](int kt, f32x16 (&s)[2], u32x4 (&pb)[4]) {
     st.mask(s, kt * kPfKTile, wq0, qi, len, a.causal, hh);
-    st.softmax(s, pb, a.scale_log2);
+    st.softmax(s, pb, a.scale_log2, kt == 0);
   };
   // K_{j+1} and V_j (read from slot 2j + 2 on) are loaded in slot 2j, whose
   // stages were last read in slot 2j - 1

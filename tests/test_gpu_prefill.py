@@ -349,3 +349,19 @@ def test_job_search_sequence_counts(n, Hq, Hkv):
     out = A.varlen_prefill_attention(q, k, v, cut, max(lens), 0.1, True)
     _check(out, q, k, v, cu, 0.1, True, torch.bfloat16)
     assert torch.equal(out, A.varlen_prefill_attention(q, k, v, cut, max(lens) + 200, 0.1, True))
+
+
+@pytest.mark.parametrize("top", [200, 1600])  # the four-wave and the ping-pong kernel
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+def test_first_tile_sets_the_maximum(top, causal, sign):
+    """Scores that rise (or fall) by hundreds from the first key tile to the
+    later ones: the maximum the first tile sets is overtaken (or stands)."""
+    lens = [top, 64, 65, 1, 129]
+    cu, q, k, v = _packed(lens, 4, 2, 128, torch.float16, 31)
+    for b, n in enumerate(lens):
+        ramp = sign * (torch.arange(n, device="cuda") // 64).to(k.dtype) / 16
+        k[int(cu[b]):int(cu[b]) + n] += ramp[:, None, None]
+    q.abs_()
+    out = A.varlen_prefill_attention(q, k, v, torch.from_numpy(cu).cuda(), top, 0.5, causal)
+    _check(out, q, k, v, cu, 0.5, causal, torch.float16)
