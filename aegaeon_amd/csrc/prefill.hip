@@ -566,6 +566,7 @@ __device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds,
     if (mine(kt)) pv(pb);
   }
   // the K stages: every wave is past its last read of them
+  static_assert(kShortWaves * kUnitQ <= 2 * kPfKTile, "the outputs fit the K stages");
   st.store(a, lds + w * (kUnitQ * RB), h, s0, len, wq0);
 }
 
@@ -744,6 +745,7 @@ __device__ __forceinline__ void attend_long(const PrefillArgs& a, uint8_t* lds, 
     }
     if (n_kt - 1 <= jw) pv(n_kt - 1, pb);  // slot 2 n_kt
     PF_BARRIER();
+    static_assert(kLongWaves / 2 * kUnitQ * D * 2 <= 2 * K_BYTES, "a half's outputs fit");
     // slot 2 n_kt + 1: the outputs, through the K stages (last read in slot
     // 2 n_kt - 1), while the other half runs its last P.V
     st.store(a, lds + w * (kUnitQ * D * 2), h, s0, len, wq0);
