@@ -234,16 +234,18 @@ __device__ __forceinline__ int4 continued_desc(int b, int grp, int64_t w0, int64
 }
 
 // A plan indexes the merge descriptors by (kv-head group, sequence) when
-// those, with kPlanHelpers to share the merges of long sequences, are no more
+// those, with plan_helpers to share the merges of long sequences, are no more
 // than the ranges, so that the combine grid is that much smaller (the
 // Qwen2.5-7B heads, 128 sequences: 160 descriptors against 256, 0.8 us per layer);
 // otherwise, and without a plan, by the range that continues the sequence.
-constexpr int kPlanHelpers = 32;
+constexpr int kPlanHelpers = 32;  // of groups of four heads, whose every descriptor has four
+                                  // workgroups of the combine grid; more of smaller groups
+inline int32_t plan_helpers(int32_t heads) { return kPlanHelpers * (kWaves / heads); }
 // Long sequences of one launch: each takes more than kMergeAlone - 1 ranges
 // beyond its first, and a range continues at most one sequence.
 constexpr int kMaxLong = kMaxRanges / kMergeAlone + 1;
-inline bool desc_per_sequence(int64_t batch, int64_t n_groups, int64_t n_ranges) {
-  return batch * n_groups + kPlanHelpers <= n_ranges;
+inline bool desc_per_sequence(int64_t batch, int64_t n_groups, int64_t n_ranges, int32_t heads) {
+  return batch * n_groups + plan_helpers(heads) <= n_ranges;
 }
 
 // Decode plan, in one device buffer: per range a record of 8
@@ -1101,6 +1103,7 @@ struct PlanArgs {
   int32_t n_groups;
   int32_t n_ranges;
   int32_t desc_per_seq;  // descriptors indexed by grp * batch + b (else by range)
+  int32_t helpers;       // descriptors after those, dealt over the long sequences
   int32_t range_wgs;     // workgroups that take the ranges
   int32_t* wg;
   int4* desc;
@@ -1199,7 +1202,7 @@ __global__ __launch_bounds__(64 * kWaves) void decode_plan_kernel(PlanArgs p) {
                     : -1;
   }
   if (!p.desc_per_seq) return;
-  // one descriptor per (group, sequence), then kPlanHelpers dealt over the
+  // one descriptor per (group, sequence), then the helpers dealt over the
   // long sequences
   const int n = p.n_groups * p.batch;
   if (threadIdx.x == 0) s_nlong = 0;
@@ -1221,15 +1224,16 @@ __global__ __launch_bounds__(64 * kWaves) void decode_plan_kernel(PlanArgs p) {
   }
   __syncthreads();
   const int R = s_nlong;
-  for (int x = threadIdx.x; x < R + kPlanHelpers; x += blockDim.x) {
+  for (int x = threadIdx.x; x < R + p.helpers; x += blockDim.x) {
     // long sequence x itself, or helper i, which is number 1 + i / R of its
     const int i = x - R, r = R == 0 ? 0 : i < 0 ? x : i % R;
     const int at = R > 0 && i < 0 ? s_long[r].x : n + i;
     int4 d = no_merge();
     if (R > 0) {
       const int4 l = s_long[r];
-      const int nh = 1 + (kPlanHelpers - r + R - 1) / R;
-      d = merge_desc(l.x % p.batch, l.x / p.batch, l.y, l.z, i < 0 ? 0 : 1 + i / R, nh);
+      const int nh = min(kMaxHelpers, 1 + (p.helpers - r + R - 1) / R);
+      const int k = i < 0 ? 0 : 1 + i / R;
+      if (k < nh) d = merge_desc(l.x % p.batch, l.x / p.batch, l.y, l.z, k, nh);
     }
     p.desc[at] = d;
   }
@@ -1302,12 +1306,17 @@ __device__ __forceinline__ int64_t new_row_chunks(const AttnArgs& a) {
 
 
 // The merge of a sequence of more than kMergeAlone pieces: the nh workgroups
-// (of one kv head) take runs of kMergeCols float4 columns (one 128-byte line of
-// a piece) in turn; the workgroup's 32 slices of 8 threads take every 32nd
-// piece each and meet through shuffles and LDS.  The sums' order does not
-// depend on nh, so every launch form gives the same bits.
-constexpr int kMergeCols = 8;
-constexpr int kMergeSlices = 64 * kWaves / kMergeCols;
+// (of one kv head) take runs of COLS float4 columns in turn; the workgroup's
+// 256 / COLS slices of COLS threads take every (256 / COLS)th piece each and
+// meet through shuffles and LDS.  COLS is the widest of 32, 16 and 8 whose
+// slices load all pieces in one round, so that a sequence of few pieces takes
+// few runs: each is a round trip and two barriers, and many such sequences
+// leave each few workgroups.  (Runs of 8 columns for all and 32 helpers
+// whatever the group size: ten sequences of 1000 tokens of 32/4 heads 25.7 us
+// per layer, so 15.0; 24 of 8/1 heads 38.4 and 13.7.)  COLS follows from the
+// pieces alone and the sums' order does not depend on nh, so every launch form
+// gives the same bits.
+constexpr int kMergeMaxCols = 32;
 constexpr int kMergeAhead = 8;  // pieces a thread loads at once
 struct MergeState {
   float m, l;
@@ -1322,34 +1331,36 @@ struct MergeState {
     o = o * w1 + o2 * w2;
   }
 };
-template <int DT, int D>
+template <int DT, int D, int COLS>
 __device__ __forceinline__ void merge_pieces_shared(const AttnArgs& a, const int4 d,
-                                                    MergeState (*s_m)[kMergeCols]) {
+                                                    MergeState (*s_m)[kMergeMaxCols]) {
   using E = Elem<DT>;
   constexpr int D4 = D / 4;
+  constexpr int SLICES = 64 * kWaves / COLS;
   const int b = d.x, grp = d.y, npieces = d.w;
   const int h = grp * a.heads + blockIdx.y;
   if (h >= a.n_kv_heads) return;
   const int w0 = d.z & 0xffff, nh = (int)((uint32_t)d.z >> 23);
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int sl = (int)threadIdx.x / kMergeCols;
+  const int sl = (int)threadIdx.x / COLS;
+  const int items = a.group * D4;  // float4 columns of the kv head's query heads
   const int64_t slot0 = (int64_t)w0 + (int64_t)grp * a.batch + b;
   const auto mlr = byte_range(reinterpret_cast<const uint8_t*>(a.part_ml), a.ml_bytes);
   const auto por = byte_range(reinterpret_cast<const uint8_t*>(a.part_o), a.o_bytes);
   const uint32_t ml_step = (uint32_t)a.hpg * 8u, o_step = (uint32_t)a.hpg * D * 4u;
-  for (int c = (d.z >> 16) & 0x7f; c < a.group * D4 / kMergeCols; c += nh) {
-    const int it = kMergeCols * c + (int)threadIdx.x % kMergeCols;
+  for (int c = (d.z >> 16) & 0x7f; c < (items + COLS - 1) / COLS; c += nh) {
+    const int it = COLS * c + (int)threadIdx.x % COLS;
     const int64_t pidx0 = slot0 * a.hpg + blockIdx.y * a.group + it / D4;
     const int col = 4 * (it % D4);
     const uint32_t ml_off = (uint32_t)(pidx0 * 8), o_off = (uint32_t)((pidx0 * D + col) * 4);
     MergeState st{-INFINITY, 0.f, f32x4{0.f, 0.f, 0.f, 0.f}};
-    for (int s0 = sl; s0 < npieces; s0 += kMergeAhead * kMergeSlices) {
+    for (int s0 = sl; s0 < npieces; s0 += kMergeAhead * SLICES) {
       float2 ml[kMergeAhead];
       f32x4 po[kMergeAhead];
 #pragma unroll
       for (int u = 0; u < kMergeAhead; ++u) {
-        const int s = s0 + u * kMergeSlices;
-        const bool ok = s < npieces;  // else past the ranges: zeros, no access
+        const int s = s0 + u * SLICES;
+        const bool ok = s < npieces && it < items;  // else past the ranges: zeros, no access
         const u32x2 mw = __builtin_amdgcn_raw_buffer_load_b64(
             mlr, ok ? ml_off + (uint32_t)s * ml_step : kPastRange, 0, 0);
         const u32x4 ow = __builtin_amdgcn_raw_buffer_load_b128(
@@ -1371,14 +1382,14 @@ __device__ __forceinline__ void merge_pieces_shared(const AttnArgs& a, const int
       st.add(mn, lt, o);
     }
 #pragma unroll
-    for (int x = kMergeCols; x < 64; x <<= 1) {
+    for (int x = COLS; x < 64; x <<= 1) {
       const f32x4 o = {__shfl_xor(st.o[0], x), __shfl_xor(st.o[1], x), __shfl_xor(st.o[2], x),
                        __shfl_xor(st.o[3], x)};
       st.add(__shfl_xor(st.m, x), __shfl_xor(st.l, x), o);
     }
-    if (lane < kMergeCols) s_m[wave][lane] = st;
+    if (lane < COLS) s_m[wave][lane] = st;
     __syncthreads();  // c is uniform over the workgroup
-    if (threadIdx.x < kMergeCols) {
+    if (threadIdx.x < COLS && it < items) {
       st = s_m[0][lane];
 #pragma unroll
       for (int w = 1; w < kWaves; ++w) st.add(s_m[w][lane].m, s_m[w][lane].l, s_m[w][lane].o);
@@ -1463,7 +1474,7 @@ __device__ __forceinline__ void merge_pieces(const AttnArgs& a, const int4 d) {
 
 template <int DT, int D, int KI, int PB>
 __global__ __launch_bounds__(64 * kWaves) void attention_combine_kernel(AttnArgs a) {
-  __shared__ MergeState s_m[kWaves][kMergeCols];
+  __shared__ MergeState s_m[kWaves][kMergeMaxCols];
   const int4 d = a.desc[blockIdx.x];
   // an appending call: this thread's first new-row chunk, loaded ahead of the merge
   const int64_t total = a.knew ? new_row_chunks<D>(a) : 0;
@@ -1478,8 +1489,10 @@ __global__ __launch_bounds__(64 * kWaves) void attention_combine_kernel(AttnArgs
     if (a.plan_last) blk0 = a.plan_last[r.b];
   }
   if (d.x >= 0) {  // uniform over the workgroup
-    if (d.w > kMergeAlone) merge_pieces_shared<DT, D>(a, d, s_m);
-    else merge_pieces<DT, D, KI, PB>(a, d);
+    if (d.w <= kMergeAlone) merge_pieces<DT, D, KI, PB>(a, d);
+    else if (d.w <= kMergeAhead * 256 / 32) merge_pieces_shared<DT, D, 32>(a, d, s_m);
+    else if (d.w <= kMergeAhead * 256 / 16) merge_pieces_shared<DT, D, 16>(a, d, s_m);
+    else merge_pieces_shared<DT, D, 8>(a, d, s_m);
   }
   if (c0 < total) {
     const NewRowChunk<D> r(a, c0);
@@ -1657,7 +1670,8 @@ int run_attention(void* out, int64_t out_batch_stride, const void* q, int64_t q_
   a.knew_span = a.vnew_span = 0;
   a.n_desc = n_ranges;
   if (plan) {
-    if (desc_per_sequence(batch, n_groups, n_ranges)) a.n_desc = batch * n_groups + kPlanHelpers;
+    if (desc_per_sequence(batch, n_groups, n_ranges, heads))
+      a.n_desc = batch * n_groups + plan_helpers(heads);
     const PlanLayout pl = plan_layout(batch, n_ranges, nblk_max);
     if (plan_bytes < (uint64_t)pl.total) return AEGKV_ERR_INVALID_ARG;
     if (!aligned16(plan)) return AEGKV_ERR_MISALIGNED;
@@ -1916,7 +1930,8 @@ int aegkv_paged_decode_plan(const int32_t* block_tables, int32_t max_blocks,
   p.max_seq_len = max_seq_len;
   p.n_groups = (n_kv_heads + heads - 1) / heads;
   p.n_ranges = n_ranges;
-  p.desc_per_seq = desc_per_sequence(batch, p.n_groups, n_ranges) ? 1 : 0;
+  p.desc_per_seq = desc_per_sequence(batch, p.n_groups, n_ranges, heads) ? 1 : 0;
+  p.helpers = plan_helpers(heads);
   p.wg = reinterpret_cast<int32_t*>(pb + pl.wg);
   p.desc = reinterpret_cast<int4*>(pb + pl.desc);
   p.first = reinterpret_cast<int32_t*>(pb + pl.first);

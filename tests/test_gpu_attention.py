@@ -986,3 +986,32 @@ def test_kv_head_counts_not_of_four(device, Hq, Hkv, D, nwg):
                                        ml, n_workgroups=nwg, plan=pl, key=key, value=val)
         assert np.array_equal(to_bits(got), to_bits(want))
         assert np.array_equal(to_bits(k3), to_bits(k2)) and np.array_equal(to_bits(v3), to_bits(v2))
+
+
+@pytest.mark.parametrize("Hq,Hkv,D", [(28, 4, 128), (7, 1, 64), (1, 1, 64), (3, 3, 64),
+                                      (16, 1, 128), (6, 2, 256)])
+@pytest.mark.parametrize("lens,nwg", [
+    ([4800], 64), ([4800], 65), ([4800], 128), ([4800], 129), ([4800], 300),
+    ([800] * 12, 300), ([800] * 12, 130), ([4000, 800] * 4, 160)])
+def test_merge_runs_of_columns(device, Hq, Hkv, D, lens, nwg):
+    """A shared merge takes runs of 32, 16 or 8 columns by its number of
+    pieces: both sides of each change, head shapes whose columns are no whole
+    number of runs (7 or 3 rows of 16 at D = 64) or less than one, many long
+    sequences that share the helpers; planned and unplanned bit for bit.  In
+    fp16, whose rounding (at most 2^-11 of a value) keeps the relative error of
+    as few as 64 outputs under the bar; bf16's (2^-8) does so on average only."""
+    rng = np.random.default_rng(nwg + D + len(lens))
+    lens, tables, padded, q, kc, vc = _setup(rng, lens, Hq, Hkv, D, "fp16")
+    scale = 1.0 / math.sqrt(D)
+    dev = lambda x: to_device_bits(x, "fp16", device)  # noqa: E731
+    bt = torch.from_numpy(padded).to(device)
+    sl = torch.from_numpy(lens.astype(np.int32)).to(device)
+    ml = int(lens.max())
+    args = (dev(q), dev(kc), dev(vc))
+    one = A.paged_decode_attention(*args, bt, sl, scale, ml, n_workgroups=nwg)
+    plan = A.DecodePlan(bt, sl, ml, Hkv, nwg)
+    two = A.paged_decode_attention(*args, None, None, scale, ml, n_workgroups=nwg, plan=plan)
+    ref = ko.paged_decode_attention(ko.bits_to_float(q, "fp16"), ko.bits_to_float(kc, "fp16"),
+                                    ko.bits_to_float(vc, "fp16"), padded, lens, scale)
+    _check(to_bits(one), ref, "fp16")
+    assert np.array_equal(to_bits(one), to_bits(two))
