@@ -8,8 +8,8 @@
 // position P = grp * W + cum[b] + kSegmentCost + j for block j of sequence b,
 // W = sum_b (ceil(len_b / 16) + kSegmentCost).  One workgroup of four waves per
 // CU takes an equal contiguous range of positions (with 2 or 1 heads per group,
-// 2 or 4 consecutive ranges), so every CU does the same work in a
-// single round, and consecutive workgroups land on different XCDs (workgroups
+// up to 2 or 4 of them: RangeRule), so every CU does the same work in a
+// single round, and consecutive ranges land on different XCDs (workgroups
 // are dealt to the XCDs round-robin).  Each workgroup computes the prefix sums of
 // the batch itself (into LDS) and walks its range; a range may cut sequences,
 // whose pieces write fp32 partials (unnormalised O, running max in log2
@@ -29,8 +29,9 @@
 // one CU ~10 us more, against ~3.6 us for this second launch.)
 //
 // Inside a workgroup of group size H, wave w handles kv head grp * H + w % H
-// over range w / H of the workgroup, and all G = Hq / Hkv query heads of that kv head are processed together, so each K/V
-// byte is read from HBM exactly once per decode step.  A wave streams the
+// over range w / H of the workgroup, and all G = Hq / Hkv query heads of that
+// kv head are processed together, so each K/V byte is read from HBM exactly
+// once per decode step.  A wave streams the
 // blocks of its whole range through one register pipeline, across sequence
 // boundaries, and keeps the pieces it finishes in LDS until the stream ends
 // (attend_items); one piece per sequence start and a pipeline drain per
@@ -111,6 +112,40 @@ inline int heads_per_group(int32_t n_kv_heads) {
   if (n_kv_heads % 4 == 0 || n_kv_heads > 63) return 4;
   return n_kv_heads % 2 == 0 ? 2 : 1;
 }
+
+// Ranges in use.  Groups of 2 or 1 heads have two or four ranges per
+// workgroup: range r is the (r / n_wg)-th of workgroup r % n_wg.  Always in use
+// are as many as make a range no longer than one of groups of four heads (one
+// per workgroup for 1 and 2 kv heads); a second, third or fourth one of every
+// workgroup joins when the batch's positions leave each range the counts below,
+// under which more pieces to merge and more starts cost what the waves gain.
+// All workgroups take as many: those with one wave more would end last (14/2
+// heads, 64 sequences: a second range on a third of them 22.0 us).  Per layer,
+// 1000 tokens each: 8/1 heads of 128, 32 sequences: one range 12.5 us,
+// four 14.6; 64: 16.8, two 13.9, four 15.7; 96: two 16.8, four 18.0; 192: one
+// 34.5, four 24.8.  14/2 heads of 128, 48: one 16.6, two 17.7; 128: 28.2 and
+// 28.6; 256: 47.4 and 47.2, of 64, 400: 84 and 53.
+struct RangeRule {
+  int32_t n_wg, least;  // ranges per step, and always in use
+  int64_t join[3];      // positions from which 2, 3 and 4 per workgroup are
+};
+inline RangeRule range_rule(int32_t n_wg, int32_t n_kv_heads, int32_t heads) {
+  const int32_t n_groups = (n_kv_heads + heads - 1) / heads;
+  RangeRule r;
+  r.n_wg = n_wg;
+  r.least = (int32_t)((int64_t)n_wg * n_groups / ((n_kv_heads + kWaves - 1) / kWaves));
+  for (int k = 2; k <= kWaves; ++k) {
+    const int64_t per_range = heads == 2 ? (n_groups == 1 ? 24 : 12) : k == 2 ? 6 : 12;
+    r.join[k - 2] = k * heads <= kWaves ? per_range * k * n_wg : INT64_MAX;
+  }
+  return r;
+}
+__device__ __forceinline__ int64_t active_ranges(const RangeRule& r, int64_t total) {
+  const int per_wg = 1 + (total >= r.join[0]) + (total >= r.join[1]) + (total >= r.join[2]);
+  // with fewer positions than that one each, so that no range is empty
+  return min(total, (int64_t)max(r.least, r.n_wg * per_wg));
+}
+
 constexpr float kRescaleSlack = 8.f;  // log2 headroom of the lazy softmax rescale
 
 template <int DT>
@@ -173,8 +208,9 @@ struct AttnArgs {
   int32_t hpg;       // query heads per group: heads * group
   int32_t n_groups;  // ceil(n_kv_heads / heads)
   int32_t n_wg;      // workgroups of the main kernel
-  int32_t splits;    // ranges per workgroup: kWaves / heads
-  int32_t n_ranges;  // n_wg * splits
+  int32_t heads_log2;  // log2(heads)
+  int32_t n_ranges;  // n_wg * kWaves / heads
+  RangeRule ranges;  // how many of them take part
   float scale_log2;  // softmax scale * log2(e)
   int32_t max_seq_len;  // host bound; longer device lengths are clamped to it
   uint16_t* out;
@@ -1011,7 +1047,8 @@ paged_decode_attention_kernel(AttnArgs a) {
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = uni(tid >> 6);
   // the wave's range and its kv head within a group
-  const int range = (int)blockIdx.x * a.splits + wave / a.heads, hl = wave % a.heads;
+  const int range = (int)blockIdx.x + a.n_wg * (wave >> a.heads_log2);
+  const int hl = wave & (a.heads - 1);
 
   // A planned range's record and the block ids of its first 64 items,
   // loaded before the scan so that they arrive while it runs.
@@ -1055,9 +1092,7 @@ paged_decode_attention_kernel(AttnArgs a) {
   }
   const int64_t W = s_cum[a.batch];
   const int64_t total = W * a.n_groups;
-  // With fewer positions than ranges only the first `total` take part, so
-  // that every range is non-empty.
-  const int64_t n_act = min((int64_t)a.n_ranges, total);
+  const int64_t n_act = active_ranges(a.ranges, total);
   if (range >= n_act) {
     if (hl == 0 && lane == 0) a.desc[range] = no_merge();
     return;
@@ -1102,6 +1137,7 @@ struct PlanArgs {
   int32_t max_seq_len;
   int32_t n_groups;
   int32_t n_ranges;
+  RangeRule ranges;
   int32_t desc_per_seq;  // descriptors indexed by grp * batch + b (else by range)
   int32_t helpers;       // descriptors after those, dealt over the long sequences
   int32_t range_wgs;     // workgroups that take the ranges
@@ -1134,7 +1170,7 @@ __global__ __launch_bounds__(64 * kWaves) void decode_plan_kernel(PlanArgs p) {
   const int64_t W = s_cum[p.batch];
   const int items = s_bcum[p.batch];
   const int64_t total = W * p.n_groups;
-  const int64_t n_act = min((int64_t)p.n_ranges, total);
+  const int64_t n_act = active_ranges(p.ranges, total);
   const int lane = threadIdx.x & 63, wave = uni(threadIdx.x >> 6);
   // item i's block id and new-row tag: an appending call's new row is the last
   // attended token, unless the sequence is longer than the bound (its new row
@@ -1655,8 +1691,9 @@ int run_attention(void* out, int64_t out_batch_stride, const void* q, int64_t q_
   a.hpg = heads * group;
   a.n_groups = n_groups;
   a.n_wg = n_wg;
-  a.splits = kWaves / heads;
+  a.heads_log2 = heads == 4 ? 2 : heads - 1;
   a.n_ranges = n_ranges;
+  a.ranges = range_rule(n_wg, n_kv_heads, heads);
   a.scale_log2 = scale * 1.4426950408889634f;
   a.max_seq_len = max_seq_len;
   a.q_bstride = q_batch_stride;
@@ -1930,6 +1967,7 @@ int aegkv_paged_decode_plan(const int32_t* block_tables, int32_t max_blocks,
   p.max_seq_len = max_seq_len;
   p.n_groups = (n_kv_heads + heads - 1) / heads;
   p.n_ranges = n_ranges;
+  p.ranges = range_rule(n_wg, n_kv_heads, heads);
   p.desc_per_seq = desc_per_sequence(batch, p.n_groups, n_ranges, heads) ? 1 : 0;
   p.helpers = plan_helpers(heads);
   p.wg = reinterpret_cast<int32_t*>(pb + pl.wg);

@@ -1015,3 +1015,44 @@ def test_merge_runs_of_columns(device, Hq, Hkv, D, lens, nwg):
                                     ko.bits_to_float(vc, "fp16"), padded, lens, scale)
     _check(to_bits(one), ref, "fp16")
     assert np.array_equal(to_bits(one), to_bits(two))
+
+
+@pytest.mark.parametrize("Hq,Hkv,D,blocks", [
+    (7, 1, 128, [46, 47, 142, 143, 190, 191]),  # a second range per workgroup at 48 positions,
+    (4, 1, 256, [46, 47, 190, 191]),            # a third at 144, a fourth at 192
+    (14, 2, 128, [190, 191]), (2, 2, 64, [190, 191]),   # a second at 192
+    (6, 6, 64, [30, 31, 32]), (12, 6, 128, [30, 31]),   # three groups: at 96, of least 6
+    (5, 5, 64, [27, 28, 37, 38])])                      # five groups: at 144 and 192, least 10
+def test_ranges_in_use(device, Hq, Hkv, D, blocks):
+    """Both sides of the positions from which a workgroup's further ranges
+    are used (four workgroups; a sequence of n blocks holds n + 1 positions per
+    group), as one sequence and as several: planned, unplanned and appending."""
+    rng = np.random.default_rng(Hq + D)
+    scale = 1.0 / math.sqrt(D)
+    dev = lambda x: to_device_bits(x, "fp16", device)  # noqa: E731
+    for n in blocks:
+        for lens in ([16 * n - 3], [16 * (n - 10), 0, 80, 33]):  # 9 blocks and 2 positions more
+            lens, tables, padded, q, kc, vc = _setup(rng, lens, Hq, Hkv, D, "fp16")
+            bt = torch.from_numpy(padded).to(device)
+            sl = torch.from_numpy(lens.astype(np.int32)).to(device)
+            ml = int(lens.max())
+            dq, dk, dv = dev(q), dev(kc), dev(vc)
+            one = A.paged_decode_attention(dq, dk, dv, bt, sl, scale, ml, n_workgroups=4)
+            ref = ko.paged_decode_attention(ko.bits_to_float(q, "fp16"),
+                                            ko.bits_to_float(kc, "fp16"),
+                                            ko.bits_to_float(vc, "fp16"), padded, lens, scale)
+            _check(to_bits(one), ref, "fp16")
+            plan = A.DecodePlan(bt, sl, ml, Hkv, 4)
+            two = A.paged_decode_attention(dq, dk, dv, None, None, scale, ml, n_workgroups=4,
+                                           plan=plan)
+            assert np.array_equal(to_bits(one), to_bits(two))
+            # appending the rows the cache already holds changes neither
+            last = [(t[(n - 1) // 16], (n - 1) % 16) if n else (0, 0)
+                    for t, n in zip(tables, lens.tolist())]
+            key = dev(np.stack([kc[b, o] for b, o in last]))
+            val = dev(np.stack([vc[b, o] for b, o in last]))
+            k2, v2 = dk.clone(), dv.clone()
+            got = A.paged_decode_attention(dq, k2, v2, None, None, scale, ml, n_workgroups=4,
+                                           plan=plan, key=key, value=val)
+            assert np.array_equal(to_bits(got), to_bits(one))
+            assert torch.equal(k2, dk) and torch.equal(v2, dv)
