@@ -103,13 +103,29 @@ template <int D>
 constexpr int pipeline_depth() { return D >= 256 ? 2 : 3; }
 
 // kv heads of a workgroup's group, one per wave; the 4 / heads waves of each
-// head take ranges of their own.  The largest of 4, 2, 1 that divides the kv
-// heads, so that no wave idles (7 query heads over one kv head, 256 sequences
-// of 1000 tokens: 42.4 us per layer with one wave of four busy, 26.0
-// with four ranges); above 63 kv heads an idle wave or two per group of four
-// matter less than the range arithmetic's bound (positions_fit).
+// head take ranges of their own.  Four, unless that leaves one wave in 20 or
+// more without a head; then the largest of 2 and 1 that divides the kv heads.
+// Groups of four against smaller ones, us per layer of a full chip (the kv
+// bytes of 80,000-400,000 tokens), head dim 128 and 64:
+//   kv heads      1          2          3          5          6          7
+//   128       46.5 30.1  103.2 95.2  38.5 39.5  64.7 49.9  65.5 56.8  46.6 44.0
+//   64        22.8 14.5   83.4 53.4  62.9 55.7  45.2 34.6  45.5 39.0  47.7 45.0
+//   kv heads      9         11         13         14         15         17
+//   128       60.8 53.7  106.4 103.9 121.2 110.7 111.3 104.9 114.4 112.1 112.8 104.6
+//   64        36.2 31.5   60.0 58.2   67.8 60.8  62.4 58.7  61.4 60.9  62.6 57.8
+//   kv heads     18         19         22         30         34         57
+//   128      103.8 99.2  104.0 103.2 105.3 101.8  87.8 84.8   81.0 78.5  75.8 75.0
+//   64        58.4 55.4   58.8 56.7   59.0 57.0  47.8 46.6   45.1 43.6  43.5 42.9
+// and with fewer idle waves, where heads of a block read at different times
+// cost about what the waves gain:
+//   kv heads     27         31         46         55         61         63
+//   128       90.3 89.3   73.9 74.7   84.7 82.6  71.9 73.2  68.3 68.5  69.1 70.6
+//   64        50.2 49.0   42.6 42.6   47.8 46.7  41.9 41.6  38.7 39.1  39.7 40.7
+// (3 heads of dim 128 are the exception; the plan does not know the dim.)  Above
+// 63 kv heads groups of four keep the range arithmetic's bound (positions_fit).
 inline int heads_per_group(int32_t n_kv_heads) {
-  if (n_kv_heads % 4 == 0 || n_kv_heads > 63) return 4;
+  const int64_t waves = ((int64_t)n_kv_heads + kWaves - 1) / kWaves * kWaves;
+  if (n_kv_heads > 63 || (waves - n_kv_heads) * 20 < waves) return 4;
   return n_kv_heads % 2 == 0 ? 2 : 1;
 }
 

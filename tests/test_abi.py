@@ -329,3 +329,15 @@ def test_signal_arrays_reject_bad_arguments_on_the_host(lib):
     assert lib.aegkv_signal_wait(addr, 1, 10, None, None) == INVALID
     raw2, addr2 = _buf(64)
     assert lib.aegkv_signal_wait(addr2, 1, 0, None, None) == INVALID  # zero timeout
+
+
+def test_kv_heads_per_group(lib):
+    """Groups of four kv heads unless one wave in 20 or more would idle, then
+    of two or one (whose plans hold two or four ranges per workgroup)."""
+    ranges = {lib.aegkv_paged_decode_plan_size(1, h, 16, 64): heads
+              for h, heads in ((4, 4), (2, 2), (1, 1))}
+    assert len(ranges) == 3
+    fewer = {h: 2 - h % 2 for h in (1, 2, 3, 5, 6, 7, 9, 10, 11, 13, 14, 15, 17, 18, 19, 21, 22,
+                                    25, 26, 29, 30, 33, 34, 37, 38, 41, 45, 49, 53, 57)}
+    for h in range(1, 80):
+        assert ranges[lib.aegkv_paged_decode_plan_size(1, h, 16, 64)] == fewer.get(h, 4), h
