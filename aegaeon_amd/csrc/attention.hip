@@ -123,9 +123,17 @@ constexpr int pipeline_depth() { return D >= 256 ? 2 : 3; }
 //   64        50.2 49.0   42.6 42.6   47.8 46.7  41.9 41.6  38.7 39.1  39.7 40.7
 // (3 heads of dim 128 are the exception; the plan does not know the dim.)  Above
 // 63 kv heads groups of four keep the range arithmetic's bound (positions_fit).
-inline int heads_per_group(int32_t n_kv_heads) {
+// Above kFewHeadsWorkgroups workgroups (a count that only a caller forces) the
+// further ranges' descriptors could take a call past the no-allocation
+// scratch that it fits with groups of four: with x bytes of partials per slot,
+// n workgroups and B sequences, four heads need at least B x more for partials
+// and fewer heads up to 48 n + 768 more for descriptors and their padding;
+// B x < 48 n + 768 and (4 n + 63 B) x >= 32 MiB, x <= 16512, only beyond it.
+constexpr int kFewHeadsWorkgroups = 480;
+inline int heads_per_group(int32_t n_kv_heads, int32_t n_wg) {
   const int64_t waves = ((int64_t)n_kv_heads + kWaves - 1) / kWaves * kWaves;
-  if (n_kv_heads > 63 || (waves - n_kv_heads) * 20 < waves) return 4;
+  if (n_kv_heads > 63 || n_wg > kFewHeadsWorkgroups || (waves - n_kv_heads) * 20 < waves)
+    return 4;
   return n_kv_heads % 2 == 0 ? 2 : 1;
 }
 
@@ -1651,7 +1659,7 @@ int run_attention(void* out, int64_t out_batch_stride, const void* q, int64_t q_
                   int32_t max_seq_len, int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim,
                   int32_t block_size, float scale, int32_t dtype, int32_t n_workgroups,
                   void* workspace, uint64_t workspace_bytes, aegkv_stream_t stream,
-                  const NewRows& nr = NewRows(), int32_t heads = 0) {
+                  const NewRows& nr = NewRows()) {
   if (batch < 0 || max_seq_len < 0 || n_q_heads <= 0 || n_kv_heads <= 0 || max_blocks < 0 ||
       n_blocks < 0 || n_workgroups < 0)
     return AEGKV_ERR_INVALID_ARG;
@@ -1684,7 +1692,7 @@ int run_attention(void* out, int64_t out_batch_stride, const void* q, int64_t q_
   int rc = workgroups_for(n_workgroups, &n_wg);
   if (rc) return rc;
   const int32_t group = n_q_heads / n_kv_heads;
-  if (heads == 0) heads = heads_per_group(n_kv_heads);  // the caller's choice needs no plan
+  const int32_t heads = heads_per_group(n_kv_heads, n_wg);
   const int32_t n_groups = (n_kv_heads + heads - 1) / heads;
   const int32_t n_ranges = n_wg * (kWaves / heads);
   if (!positions_fit(chunk, nblk_max, n_groups, n_ranges)) return AEGKV_ERR_UNSUPPORTED;
@@ -1779,9 +1787,9 @@ int run_attention(void* out, int64_t out_batch_stride, const void* q, int64_t q_
   return AEGKV_OK;
 }
 
-// Workspace bytes of one call with `heads` kv heads per group, or a status.
+// Workspace bytes of one call, or a status.
 int64_t workspace_size(int32_t batch, int32_t n_q_heads, int32_t n_kv_heads, int32_t head_dim,
-                       int32_t max_seq_len, int32_t dtype, int32_t n_workgroups, int32_t heads) {
+                       int32_t max_seq_len, int32_t dtype, int32_t n_workgroups) {
   if (batch < 0 || n_q_heads <= 0 || n_kv_heads <= 0 || n_q_heads % n_kv_heads ||
       n_workgroups < 0 || max_seq_len < 0)
     return AEGKV_ERR_INVALID_ARG;
@@ -1795,6 +1803,7 @@ int64_t workspace_size(int32_t batch, int32_t n_q_heads, int32_t n_kv_heads, int
   const int rc = workgroups_for(n_workgroups, &n_wg);
   if (rc) return rc > 0 ? AEGKV_ERR_RUNTIME : rc;
   const int32_t group = n_q_heads / n_kv_heads;
+  const int32_t heads = heads_per_group(n_kv_heads, n_wg);
   const int32_t n_groups = (n_kv_heads + heads - 1) / heads;
   const int32_t n_ranges = n_wg * (kWaves / heads);
   if (!positions_fit(chunk, ((int64_t)max_seq_len + kBlockSize - 1) / kBlockSize, n_groups,
@@ -1849,16 +1858,8 @@ int aegkv_paged_decode_attention_noalloc(void* out, int64_t out_batch_stride, co
                                          int32_t n_kv_heads, int32_t head_dim,
                                          int32_t block_size, float scale, int32_t dtype,
                                          int32_t n_workgroups, aegkv_stream_t stream) {
-  // Groups of fewer than four heads need fewer partials but more descriptors:
-  // a call that only fits the scratch with groups of four takes those.
-  int32_t heads = n_kv_heads > 0 ? heads_per_group(n_kv_heads) : kWaves;
-  int64_t need = workspace_size(batch, n_q_heads, n_kv_heads, head_dim, max_seq_len, dtype,
-                                n_workgroups, heads);
-  if (need > (int64_t)kScratchBytes && heads < kWaves) {
-    heads = kWaves;
-    need = workspace_size(batch, n_q_heads, n_kv_heads, head_dim, max_seq_len, dtype,
-                          n_workgroups, heads);
-  }
+  const int64_t need = workspace_size(batch, n_q_heads, n_kv_heads, head_dim, max_seq_len, dtype,
+                                      n_workgroups);
   if (need < 0) return (int)need;
   if ((uint64_t)need > kScratchBytes) return AEGKV_ERR_SCRATCH;
   if (batch == 0) return AEGKV_OK;
@@ -1869,16 +1870,14 @@ int aegkv_paged_decode_attention_noalloc(void* out, int64_t out_batch_stride, co
   return run_attention(out, out_batch_stride, q, q_batch_stride, key_cache, value_cache,
                        cache_block_stride, n_blocks, block_tables, max_blocks, nullptr, 0,
                        seq_lens, batch, max_seq_len, n_q_heads, n_kv_heads, head_dim,
-                       block_size, scale, dtype, n_workgroups, ws, kScratchBytes, stream,
-                       NewRows(), heads);
+                       block_size, scale, dtype, n_workgroups, ws, kScratchBytes, stream);
 }
 
 int64_t aegkv_paged_decode_attention_workspace_size(int32_t batch, int32_t n_q_heads,
                                                      int32_t n_kv_heads, int32_t head_dim,
                                                      int32_t max_seq_len, int32_t dtype,
                                                      int32_t n_workgroups) {
-  return workspace_size(batch, n_q_heads, n_kv_heads, head_dim, max_seq_len, dtype, n_workgroups,
-                        heads_per_group(n_kv_heads));
+  return workspace_size(batch, n_q_heads, n_kv_heads, head_dim, max_seq_len, dtype, n_workgroups);
 }
 
 int aegkv_paged_decode_attention(void* out, int64_t out_batch_stride, const void* q,
@@ -1949,7 +1948,7 @@ int64_t aegkv_paged_decode_plan_size(int32_t batch, int32_t n_kv_heads, int32_t 
   const int rc = workgroups_for(n_workgroups, &n_wg);
   if (rc) return rc > 0 ? AEGKV_ERR_RUNTIME : rc;
   const int64_t nblk_max = ((int64_t)max_seq_len + kBlockSize - 1) / kBlockSize;
-  const int32_t heads = heads_per_group(n_kv_heads);
+  const int32_t heads = heads_per_group(n_kv_heads, n_wg);
   const int32_t n_ranges = n_wg * (kWaves / heads);
   if (!positions_fit(batch, nblk_max, (n_kv_heads + heads - 1) / heads, n_ranges))
     return AEGKV_ERR_UNSUPPORTED;
@@ -1971,7 +1970,7 @@ int aegkv_paged_decode_plan(const int32_t* block_tables, int32_t max_blocks,
   int n_wg = 0;
   int rc = workgroups_for(n_workgroups, &n_wg);
   if (rc) return rc;
-  const int32_t heads = heads_per_group(n_kv_heads);
+  const int32_t heads = heads_per_group(n_kv_heads, n_wg);
   const int32_t n_ranges = n_wg * (kWaves / heads);
   const PlanLayout pl = plan_layout(batch, n_ranges, nblk_max);
   uint8_t* pb = static_cast<uint8_t*>(plan);

@@ -334,10 +334,47 @@ def test_signal_arrays_reject_bad_arguments_on_the_host(lib):
 def test_kv_heads_per_group(lib):
     """Groups of four kv heads unless one wave in 20 or more would idle, then
     of two or one (whose plans hold two or four ranges per workgroup)."""
-    ranges = {lib.aegkv_paged_decode_plan_size(1, h, 16, 64): heads
+    ranges = {lib.aegkv_paged_decode_plan_size(1, h, 16, 64): heads  # forced: no GPU needed
               for h, heads in ((4, 4), (2, 2), (1, 1))}
     assert len(ranges) == 3
     fewer = {h: 2 - h % 2 for h in (1, 2, 3, 5, 6, 7, 9, 10, 11, 13, 14, 15, 17, 18, 19, 21, 22,
                                     25, 26, 29, 30, 33, 34, 37, 38, 41, 45, 49, 53, 57)}
     for h in range(1, 80):
         assert ranges[lib.aegkv_paged_decode_plan_size(1, h, 16, 64)] == fewer.get(h, 4), h
+
+
+def _workspace_groups_of_four(batch, hq, hkv, dim, n_wg):
+    """Descriptors and partials of a launch with groups of four kv heads."""
+    up = lambda x: (x + 255) // 256 * 256  # noqa: E731
+    group, n_groups, chunk = hq // hkv, -(-hkv // 4), min(batch, 2048)
+    slots = n_wg + n_groups * chunk
+    return up(16 * n_wg) + up(8 * slots * 4 * group) + up(4 * slots * 4 * group * dim)
+
+
+@pytest.mark.parametrize("n_wg", [1, 16, 256, 400, 480, 481, 1000, 7860, 7875, 8192])
+def test_no_alloc_scratch_holds_what_groups_of_four_need(lib, n_wg):
+    """The no-allocation call is refused exactly when the workspace query
+    exceeds its 32 MiB, and groups of fewer heads take no call past that which
+    groups of four keep under it (the largest batches that they do)."""
+    limit = 32 << 20
+    raw, p = _buf(64)
+    for hkv in (1, 2, 3, 5, 6, 7, 9, 14, 18, 22, 30, 57, 63):
+        for group in (1, 2, 3, 4, 7, 16):
+            for dim in (64, 128, 256):
+                hq = hkv * group
+                fits = [b for b in (1, 2, 3, 5, 16, 64, 200, 700, 1500, 2048)
+                        if _workspace_groups_of_four(b, hq, hkv, dim, n_wg) <= limit]
+                if not fits:
+                    continue
+                top = fits[-1]
+                while top < 2048 and _workspace_groups_of_four(top + 1, hq, hkv, dim,
+                                                               n_wg) <= limit:
+                    top += 1
+                for b in (fits[0], top, top + 1):
+                    need = lib.aegkv_paged_decode_attention_workspace_size(b, hq, hkv, dim, 16, 0,
+                                                                           n_wg)
+                    assert need > 0 and (b > top or need <= limit), (hkv, group, dim, b, need)
+                    rc = lib.aegkv_paged_decode_attention_noalloc(
+                        p, hq * dim, p, hq * dim, p, p, 16 * hkv * dim, 1, None, 1, p, b, 16, hq,
+                        hkv, dim, 16, 1.0, 0, n_wg, None)
+                    assert rc == (-11 if need > limit else INVALID), (hkv, group, dim, b, need)
