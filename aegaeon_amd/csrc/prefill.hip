@@ -60,9 +60,14 @@
 // i to XCD i % 8: with a multiple of 8 pairs of one length, XCD x runs every
 // tile of the x-th eighth of the pairs, whose K and V its L2 keeps (1 x 4096
 // tokens of 40 heads: 193.5 us against 197.4 with the pairs dealt in turn), and
-// fewer pairs spread evenly over the XCDs.  Prompts of different lengths: each wave finds job i
-// among the tiles that exist (pick_job), so no workgroup is launched for an
-// empty tile (48 prompts of 25-766 tokens: 5900 of 9200 workgroups were).
+// fewer pairs spread evenly over the XCDs.  Prompts of different lengths: each
+// wave finds job i among the tiles that exist (pick_job), so no workgroup is
+// launched for an empty tile (48 prompts of 25-766 tokens: 5900 of 9200
+// workgroups were).  More of them than a wave searches, and fewer tokens than
+// 90% of the bound: the pairs are dealt in turn, as an eighth of them could be
+// all the long ones (320 prompts of 16-1024 tokens sorted by length, 32/4
+// heads: eighths 1189 us, in turn 418; unsorted 472 and 429; of one length 341
+// and 349).
 #include <algorithm>
 #include <cmath>
 
@@ -165,6 +170,7 @@ struct PrefillArgs {
   int32_t n_pairs;                             // batch * n_kv_heads
   int32_t n_tiles;                             // tiles of a pair of max_seqlen tokens
   int32_t compact;                             // jobs numbered over existing tiles only
+  int32_t in_turn;                             // else: pairs dealt to the XCDs in turn
   float scale_log2;                            // softmax scale * log2(e), > 0
 };
 
@@ -425,7 +431,7 @@ __device__ __forceinline__ bool pick_job(const PrefillArgs& a, int& kvh, int& s0
   // every tile of the bound: tile n_tiles - 1 of each pair first
   const int k = a.by_pairs.div((int)i);
   int r = (int)i - k * a.n_pairs;
-  if (a.n_pairs % kXcds == 0) r = r % kXcds * (a.n_pairs / kXcds) + r / kXcds;
+  if (a.n_pairs % kXcds == 0 && !a.in_turn) r = r % kXcds * (a.n_pairs / kXcds) + r / kXcds;
   const int b = a.by_heads.div(r);
   kvh = r - b * a.n_kv_heads;
   seq_range(a, b, s0, len);
@@ -870,6 +876,7 @@ int aegkv_varlen_prefill_attention(void* out, int64_t out_token_stride, const vo
   a.by_pairs = fast_div((int32_t)n_pairs);
   a.n_tiles = (int32_t)n_tiles;
   a.compact = compact ? 1 : 0;
+  a.in_turn = total_tokens * 10 < (int64_t)batch * max_seqlen * 9 ? 1 : 0;
   a.causal = causal ? 1 : 0;
   a.scale_log2 = scale * 1.4426950408889634f;
   const uint32_t g32 = (uint32_t)grid;

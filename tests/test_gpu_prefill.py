@@ -365,3 +365,36 @@ def test_first_tile_sets_the_maximum(top, causal, sign):
     q.abs_()
     out = A.varlen_prefill_attention(q, k, v, torch.from_numpy(cu).cuda(), top, 0.5, causal)
     _check(out, q, k, v, cu, 0.5, causal, torch.float16)
+
+
+@pytest.mark.parametrize("n", [264, 320])
+@pytest.mark.parametrize("Hq,Hkv", [(3, 1), (4, 2)])
+@pytest.mark.parametrize("top", [130, 1600])  # the four-wave and the ping-pong kernel
+@pytest.mark.parametrize("ragged", [True, False])
+def test_many_prompts_over_the_xcds(n, Hq, Hkv, top, ragged):
+    """More than 256 prompts whose (prompt, kv head) pairs are a multiple of
+    the eight XCDs, sorted by length: dealt in turn where the lengths differ
+    widely, an eighth of the pairs per XCD where they nearly reach the bound
+    (some then lack the last tile).  The first 256 alone, numbered over their
+    own tiles, give the same bits; the middle and the end match the oracle."""
+    rng = np.random.default_rng(n + Hq)
+    if ragged:
+        lens = np.sort(rng.integers(0, 100, n))
+        lens[-1] = top
+    else:
+        lens = np.sort(rng.integers(top - top // 12, top + 1, n)) if top < 1000 else \
+            np.full(n, top)
+        lens[:3] = top - top // 3
+        lens[-1] = top
+    assert (n * Hkv) % 8 == 0
+    assert (int(lens.sum()) * 10 < n * top * 9) == ragged
+    cu, q, k, v = _packed(lens.tolist(), Hq, Hkv, 64, torch.bfloat16, n)
+    cu_t = torch.from_numpy(cu).cuda()
+    out = A.varlen_prefill_attention(q, k, v, cu_t, top, 0.125, True)
+    m = int(cu[256])
+    first = A.varlen_prefill_attention(q[:m], k[:m], v[:m], cu_t[:257], int(lens[:256].max()),
+                                       0.125, True)
+    assert torch.equal(first.view(torch.int16), out[:m].view(torch.int16))
+    for b0, b1 in ((n // 2, n // 2 + 4), (n - 2, n)):
+        o, e = int(cu[b0]), int(cu[b1])
+        _check(out[o:e], q[o:e], k[o:e], v[o:e], cu[b0:b1 + 1] - o, 0.125, True, torch.bfloat16)
