@@ -171,7 +171,8 @@ struct PrefillArgs {
   int32_t n_tiles;                             // tiles of a pair of max_seqlen tokens
   int32_t compact;                             // jobs numbered over existing tiles only
   int32_t in_turn;                             // else: pairs dealt to the XCDs in turn
-  float scale_log2;                            // softmax scale * log2(e), > 0
+  float scale_log2;                            // |softmax scale| * log2(e), > 0 (1 for 0)
+  int32_t scale_sign;                          // of the scale: 1, -1 or 0
 };
 
 // The wave's state for its 32 queries: lane (col = l & 31, hh = l / 32) holds
@@ -198,6 +199,19 @@ struct WaveState {
       for (int i = 0; i < 16; ++i) o[db][i] = 0.f;
     m = -INFINITY;
     lsum = 0.f;
+  }
+
+  // The softmax takes a maximum of raw scores and masks them with -inf, so its
+  // scale is positive; another one's sign goes into the loaded queries, where
+  // it is exact (scale 0: no query, every score 0).  Kernels of their own
+  // (SIGNED) do that: a test of the scale here had the compiler wait for the
+  // queries as they are loaded.
+  __device__ __forceinline__ void sign_queries(const PrefillArgs& a) {
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        qv[ks][i] = a.scale_sign < 0 ? qv[ks][i] ^ 0x80008000u : 0u;
   }
 
   // S^T of a 64-key tile from K rows at kp (pitch KPITCH bytes, this lane's
@@ -454,7 +468,7 @@ __device__ __forceinline__ bool pick_job(const PrefillArgs& a, int& kvh, int& s0
 // (the loads pick the chunk, the LDS position is the lane's): K chunk c of row
 // r at c ^ (r % 16) at D = 128, V chunk c at c ^ 4 (r % 4), so the 16 rows of a
 // K read and the 4 rows of a transposing V read hit distinct banks.
-template <int DT, int D>
+template <int DT, int D, bool SIGNED>
 __device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds, int kvh,
                                              int64_t s0, int len, int u0) {
   using E = PfOps<DT>;
@@ -555,6 +569,7 @@ __device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds,
   asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NI) : "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
+  if constexpr (SIGNED) st.sign_queries(a);
   for (int kt = 0; kt < n_kt; ++kt) {
     if (kt > 0) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's V reads
@@ -580,19 +595,19 @@ __device__ __forceinline__ void attend_short(const PrefillArgs& a, uint8_t* lds,
   st.store(a, lds + w * (kUnitQ * RB), h, s0, len, wq0);
 }
 
-template <int DT, int D>
+template <int DT, int D, bool SIGNED>
 __global__ __launch_bounds__(kShortThreads, 3) void prefill_short_kernel(PrefillArgs a) {
   // two K stages, then one V stage
   __shared__ __align__(16) uint8_t lds[3 * kPfKTile * D * 2];
   int kvh, s0, len, u0;
   if (!pick_job<kShortWaves>(a, kvh, s0, len, u0)) return;  // uniform, before any barrier
-  attend_short<DT, D>(a, lds, kvh, s0, len, u0);
+  attend_short<DT, D, SIGNED>(a, lds, kvh, s0, len, u0);
 }
 
 // ----------------------------------------------------------------- long prompts
 // Units [u0, u0 + 8) of kv head kvh of the sequence at token s0 with len
 // tokens, ping-pong between the workgroup's halves.
-template <int DT, int D>
+template <int DT, int D, bool SIGNED>
 __device__ __forceinline__ void attend_long(const PrefillArgs& a, uint8_t* lds, int kvh,
                                             int64_t s0, int len, int u0) {
   using E = PfOps<DT>;
@@ -743,6 +758,7 @@ __device__ __forceinline__ void attend_long(const PrefillArgs& a, uint8_t* lds, 
   u32x4 pb[4];
   dma_k(0);
   __syncthreads();  // waits for K_0 and the queries
+  if constexpr (SIGNED) st.sign_queries(a);
   if (half == 0) {
     for (int j = 0; j < n_kt; ++j) {
       f32x16 sc[2];  // slot 2j
@@ -781,7 +797,7 @@ __device__ __forceinline__ void attend_long(const PrefillArgs& a, uint8_t* lds, 
 #undef PF_BARRIER_LOADED
 }
 
-template <int DT, int D>
+template <int DT, int D, bool SIGNED>
 __global__ __launch_bounds__(kLongThreads) void prefill_long_kernel(PrefillArgs a) {
   constexpr int K_BYTES = kPfKTile * (D * 2 + 16);
   constexpr int V_BYTES = kPfKTile * (D * 2 + 64);
@@ -789,17 +805,22 @@ __global__ __launch_bounds__(kLongThreads) void prefill_long_kernel(PrefillArgs 
   __shared__ __align__(16) uint8_t lds[2 * K_BYTES + 2 * V_BYTES];
   int kvh, s0, len, u0;
   if (!pick_job<kLongWaves>(a, kvh, s0, len, u0)) return;  // uniform, before any barrier
-  attend_long<DT, D>(a, lds, kvh, s0, len, u0);
+  attend_long<DT, D, SIGNED>(a, lds, kvh, s0, len, u0);
 }
 
+template <int DT, int D, bool SIGNED>
+void launch_kernel(const PrefillArgs& a, bool long_prompts, uint32_t grid, hipStream_t stream) {
+  if (long_prompts)
+    hipLaunchKernelGGL((prefill_long_kernel<DT, D, SIGNED>), dim3(grid), dim3(kLongThreads), 0,
+                       stream, a);
+  else
+    hipLaunchKernelGGL((prefill_short_kernel<DT, D, SIGNED>), dim3(grid), dim3(kShortThreads), 0,
+                       stream, a);
+}
 template <int DT, int D>
 void launch_prefill(const PrefillArgs& a, bool long_prompts, uint32_t grid, hipStream_t stream) {
-  if (long_prompts)
-    hipLaunchKernelGGL((prefill_long_kernel<DT, D>), dim3(grid), dim3(kLongThreads), 0, stream,
-                       a);
-  else
-    hipLaunchKernelGGL((prefill_short_kernel<DT, D>), dim3(grid), dim3(kShortThreads), 0, stream,
-                       a);
+  if (a.scale_sign > 0) launch_kernel<DT, D, false>(a, long_prompts, grid, stream);
+  else launch_kernel<DT, D, true>(a, long_prompts, grid, stream);
 }
 
 }  // namespace
@@ -882,7 +903,8 @@ int aegkv_varlen_prefill_attention(void* out, int64_t out_token_stride, const vo
   a.compact = compact ? 1 : 0;
   a.in_turn = total_tokens * 10 < (int64_t)batch * max_seqlen * 9 ? 1 : 0;
   a.causal = causal ? 1 : 0;
-  a.scale_log2 = scale * 1.4426950408889634f;
+  a.scale_sign = scale > 0 ? 1 : scale < 0 ? -1 : 0;
+  a.scale_log2 = scale == 0 ? 1.f : std::fabs(scale) * 1.4426950408889634f;
   const uint32_t g32 = (uint32_t)grid;
   if (dtype == AEGKV_DTYPE_BF16) {
     if (head_dim == 64) launch_prefill<AEGKV_DTYPE_BF16, 64>(a, long_prompts, g32, stream);

@@ -398,3 +398,22 @@ def test_many_prompts_over_the_xcds(n, Hq, Hkv, top, ragged):
     for b0, b1 in ((n // 2, n // 2 + 4), (n - 2, n)):
         o, e = int(cu[b0]), int(cu[b1])
         _check(out[o:e], q[o:e], k[o:e], v[o:e], cu[b0:b1 + 1] - o, 0.125, True, torch.bfloat16)
+
+
+@pytest.mark.parametrize("scale", [-0.11, 0.0, -0.0, 0.11])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("top", [200, 1600])  # the four-wave and the ping-pong kernel
+@pytest.mark.parametrize("causal", [True, False])
+def test_any_finite_scale(scale, D, top, causal):
+    """A negative scale prefers the smallest products, zero weighs every key
+    alike; masked keys stay masked.  A negative scale equals the positive one
+    on negated queries bit for bit."""
+    lens = [top, 64, 1, 65, 30]
+    for dtype in (torch.bfloat16, torch.float16):
+        cu, q, k, v = _packed(lens, 4, 2, D, dtype, 43)
+        cu_t = torch.from_numpy(cu).cuda()
+        out = A.varlen_prefill_attention(q, k, v, cu_t, top, scale, causal)
+        _check(out, q, k, v, cu, scale, causal, dtype)
+        if scale:
+            neg = A.varlen_prefill_attention(-q, k, v, cu_t, top, -scale, causal)
+            assert torch.equal(out.view(torch.int16), neg.view(torch.int16))
