@@ -170,7 +170,7 @@ struct PrefillArgs {
   int32_t n_pairs;                             // batch * n_kv_heads
   int32_t n_tiles;                             // tiles of a pair of max_seqlen tokens
   int32_t compact;                             // jobs numbered over existing tiles only
-  int32_t in_turn;                             // else: pairs dealt to the XCDs in turn
+  int32_t per_xcd;                             // else: pairs per XCD (0: dealt in turn)
   float scale_log2;                            // |softmax scale| * log2(e), > 0 (1 for 0)
   int32_t scale_sign;                          // of the scale: 1, -1 or 0
 };
@@ -445,7 +445,7 @@ __device__ __forceinline__ bool pick_job(const PrefillArgs& a, int& kvh, int& s0
   // every tile of the bound: tile n_tiles - 1 of each pair first
   const int k = a.by_pairs.div((int)i);
   int r = (int)i - k * a.n_pairs;
-  if (a.n_pairs % kXcds == 0 && !a.in_turn) r = r % kXcds * (a.n_pairs / kXcds) + r / kXcds;
+  if (a.per_xcd) r = r % kXcds * a.per_xcd + r / kXcds;
   const int b = a.by_heads.div(r);
   kvh = r - b * a.n_kv_heads;
   seq_range(a, b, s0, len);
@@ -901,7 +901,9 @@ int aegkv_varlen_prefill_attention(void* out, int64_t out_token_stride, const vo
   a.by_pairs = fast_div((int32_t)n_pairs);
   a.n_tiles = (int32_t)n_tiles;
   a.compact = compact ? 1 : 0;
-  a.in_turn = total_tokens * 10 < (int64_t)batch * max_seqlen * 9 ? 1 : 0;
+  const bool in_turn =
+      n_pairs % kXcds != 0 || total_tokens * 10 < (int64_t)batch * max_seqlen * 9;
+  a.per_xcd = in_turn ? 0 : (int32_t)(n_pairs / kXcds);
   a.causal = causal ? 1 : 0;
   a.scale_sign = scale > 0 ? 1 : scale < 0 ? -1 : 0;
   a.scale_log2 = scale == 0 ? 1.f : std::fabs(scale) * 1.4426950408889634f;
