@@ -12,8 +12,10 @@ _CURRENT = nullcontext()
 
 
 def device_guard(device: torch.device):
-    """Makes ``device`` current inside the ``with`` (nothing to do when it is)."""
-    if device.index is not None and device.index == torch.cuda.current_device():
+    """Makes the GPU ``device`` current inside the ``with`` (nothing to do when
+    it is); ValueError for a device that is no GPU, also ``cpu:0``."""
+    if device.type == "cuda" and device.index is not None \
+            and device.index == torch.cuda.current_device():
         return _CURRENT
     return torch.cuda.device(device)
 
