@@ -88,6 +88,7 @@ def _prepare(ids, offsets, seq, ctx, tokens, n_tokens: int, device, block_size: 
      max_decode) = _listpack.step_counts(offsets, seq, ctx)
     if n_tokens != T:
         raise ValueError("tokens must hold every request's new tokens")
+    pad_width = max(pad_width, 0)  # decreasing offsets: the call refuses them
     B = len(seq_list)
 
     # the outputs are views of one int32 and one int64 allocation (two
