@@ -18,6 +18,7 @@ from __future__ import annotations
 import math
 import threading
 import weakref
+from contextlib import nullcontext
 from typing import Dict, Optional, Sequence, Tuple
 
 import torch
@@ -208,7 +209,7 @@ def attention_workspace(batch: int, n_q_heads: int, n_kv_heads: int, head_dim: i
                         n_workgroups: int = 0, device=None) -> Optional[torch.Tensor]:
     """A device workspace large enough for every call of these sizes (None
     when the call needs none); reusable by consecutive calls on one stream,
-    calls that may overlap (other streams) need their own."""
+    calls that may overlap (other streams, other threads) need their own."""
     dev = _gpu(device)
     n = attention_workspace_bytes(batch, n_q_heads, n_kv_heads, head_dim, max_seq_len, dtype,
                                   n_workgroups, dev)
@@ -217,19 +218,32 @@ def attention_workspace(batch: int, n_q_heads: int, n_kv_heads: int, head_dim: i
     return torch.empty(n, dtype=torch.uint8, device=dev)
 
 
-# Workspaces kept per (device, stream) for calls that bring none.
-_workspaces: Dict[Tuple[int, int], torch.Tensor] = {}
-_ws_lock = threading.Lock()
+class _StreamWorkspace:
+    """The workspace of the calls on one stream that bring none.  A call
+    enqueues a kernel that fills it and one that merges from it, and a second
+    host thread on the stream (torch's default stream is every thread's) must
+    not come between them: ``lock`` is held while a call enqueues."""
+
+    def __init__(self):
+        self.lock = threading.Lock()
+        self.buffer: Optional[torch.Tensor] = None
+
+    def at_least(self, nbytes: int, device: torch.device) -> torch.Tensor:
+        """The buffer, grown to ``nbytes`` (lock held)."""
+        if self.buffer is None or self.buffer.numel() < nbytes:
+            self.buffer = torch.empty(nbytes, dtype=torch.uint8, device=device)
+        return self.buffer
 
 
-def _cached_workspace(device: torch.device, stream: int, nbytes: int) -> torch.Tensor:
+_workspaces: Dict[Tuple[int, int], _StreamWorkspace] = {}
+_OWN_WORKSPACE = nullcontext()
+
+
+def _stream_workspace(device: torch.device, stream: int) -> _StreamWorkspace:
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
-    with _ws_lock:
-        ws = _workspaces.get(key)
-        if ws is None or ws.numel() < nbytes:
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-            _workspaces[key] = ws
-        return ws
+    ws = _workspaces.get(key)
+    # setdefault: of threads that come here together one's entry is everyone's
+    return ws if ws is not None else _workspaces.setdefault(key, _StreamWorkspace())
 
 
 def _int32_dense(t: torch.Tensor) -> torch.Tensor:
@@ -301,10 +315,11 @@ def paged_decode_attention(q: torch.Tensor, key_cache: torch.Tensor, value_cache
     views ``[N, 16, Hkv, D]``; returns ``out [B, Hq, D]`` in q's dtype.
     ``n_workgroups`` = 0 spreads the batch over one workgroup per CU; a
     positive count forces that many (same result).  ``workspace``: from
-    :func:`attention_workspace` (reusable on one stream); by default a cached
-    one per (device, stream).  ``plan``: a :class:`DecodePlan` of this step's
-    tables and lengths (then ``block_tables``/``seq_lens`` may be None, or
-    must be the tensors it was built from); the result is identical.
+    :func:`attention_workspace` (reusable on one stream, by one thread at a
+    time); by default one per (device, stream) that threads may share.
+    ``plan``: a :class:`DecodePlan` of this step's tables and lengths (then
+    ``block_tables``/``seq_lens`` may be None, or must be the tensors it was
+    built from); the result is identical.
     ``key``/``value`` ``[B, Hkv, D]``: append them first, in the same call
     (aegkv_paged_decode_attention_append): ``seq_lens[b]`` counts the new
     token, which lands at position ``seq_lens[b] - 1`` of sequence b's table
@@ -371,15 +386,14 @@ def paged_decode_attention(q: torch.Tensor, key_cache: torch.Tensor, value_cache
         if ws_bytes < 0:
             _lib.check(int(ws_bytes), "attention_workspace_bytes")
         stream = raw_stream(dev)
-        ws_ptr = None
-        if ws_bytes > 0:
-            if workspace is None:
-                workspace = _cached_workspace(dev, stream, ws_bytes)
+        shared = None  # the stream's workspace when the call brings none
+        if ws_bytes > 0 and workspace is None:
+            shared = _stream_workspace(dev, stream)
+        elif ws_bytes > 0:
             _check_on(workspace, "workspace", dev)
             if workspace.numel() * workspace.element_size() < ws_bytes:
                 raise ValueError(f"workspace holds {workspace.numel() * workspace.element_size()} "
                                  f"bytes, the call needs {ws_bytes}")
-            ws_ptr = workspace.data_ptr()
         if plan is not None and stream != plan.raw_stream:
             plan.wait_for_build(torch.cuda.current_stream(dev))
         args = (out.data_ptr(), out.stride(0), q.data_ptr(), q.stride(0))
@@ -395,8 +409,12 @@ def paged_decode_attention(q: torch.Tensor, key_cache: torch.Tensor, value_cache
             args += (bt.data_ptr(), bt.size(1))
             call = lib.aegkv_paged_decode_attention if key is None \
                 else lib.aegkv_paged_decode_attention_append
-        rc = call(*args, sl.data_ptr(), B, max_seq_len, Hq, Hkv, D, bs, float(scale), dtype,
-                  n_workgroups, ws_ptr, ws_bytes if ws_ptr else 0, stream)
+        with _OWN_WORKSPACE if shared is None else shared.lock:
+            if shared is not None:
+                workspace = shared.at_least(ws_bytes, dev)
+            rc = call(*args, sl.data_ptr(), B, max_seq_len, Hq, Hkv, D, bs, float(scale), dtype,
+                      n_workgroups, workspace.data_ptr() if ws_bytes > 0 else None, ws_bytes,
+                      stream)
     _lib.check(rc, "paged_decode_attention")
     return out
 

@@ -228,8 +228,9 @@ int aegkv_gather_tokens(const void* key_cache, const void* value_cache,
  *     aegkv_paged_decode_attention_workspace_size(...) bytes (same batch, heads,
  *     head_dim, max_seq_len, dtype, n_workgroups and device); it holds the
  *     partials of sequences that several workgroups share; its contents need
- *     no initialisation.  Calls that may run concurrently (other streams) must
- *     not share a workspace.
+ *     no initialisation.  Calls that may run concurrently (other streams), or
+ *     whose kernels may be enqueued between each other's (other host threads on
+ *     the stream), must not share a workspace.
  * Supported: block_size 16, head_dim 64/128/256, n_q_heads/n_kv_heads <= 16
  * (AEGKV_ERR_UNSUPPORTED otherwise).  Batches above 2048 sequences run as
  * consecutive launches of 2048.  seq_lens[b] == 0 yields zeros.  A block id

@@ -1056,3 +1056,42 @@ def test_ranges_in_use(device, Hq, Hkv, D, blocks):
                                            plan=plan, key=key, value=val)
             assert np.array_equal(to_bits(got), to_bits(one))
             assert torch.equal(k2, dk) and torch.equal(v2, dv)
+
+
+def test_threads_share_a_streams_workspace(device):
+    """Two host threads on the default stream, whose calls share its
+    workspace, with different cut sequences: every output equals the serial
+    one's, bit for bit (stops at the first that does not)."""
+    import threading
+    rng = np.random.default_rng(11)
+    cases = []
+    for lens, Hq, Hkv, D in (([3000, 40, 900], 28, 4, 128), ([5000, 1, 700, 2000], 8, 8, 64)):
+        lens, _, padded, q, kc, vc = _setup(rng, lens, Hq, Hkv, D, "bf16")
+        dev = lambda x: to_device_bits(x, "bf16", device)  # noqa: E731
+        cases.append((dev(q), dev(kc), dev(vc), torch.from_numpy(padded).to(device),
+                      torch.from_numpy(lens.astype(np.int32)).to(device), 1.0 / math.sqrt(D),
+                      int(lens.max())))
+    want = [A.paged_decode_attention(*c) for c in cases]
+    torch.cuda.synchronize()
+    bad, errors, stop = [], [], threading.Event()
+
+    def work(i):
+        try:
+            for _ in range(100):
+                if stop.is_set():
+                    return
+                outs = [A.paged_decode_attention(*cases[i]) for _ in range(4)]
+                if not all(torch.equal(o.view(torch.int16), want[i].view(torch.int16))
+                           for o in outs):
+                    bad.append(i)
+                    stop.set()
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+            stop.set()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors and not bad, (errors, bad)

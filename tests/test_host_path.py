@@ -1,5 +1,7 @@
-"""The host side of a launch without a GPU (the device queries are stood in
-for)."""
+"""The host side of a launch without a GPU (the device queries, and the
+library where a call would enqueue, are stood in for)."""
+import threading
+import time
 from contextlib import nullcontext
 
 import numpy as np
@@ -7,6 +9,7 @@ import pytest
 import torch
 
 from aegaeon_amd import _gpu, inputs
+from aegaeon_amd import attention as A
 from aegaeon_amd._lib import AegkvError
 
 
@@ -43,3 +46,75 @@ def test_decreasing_table_offsets_are_refused_by_the_call(monkeypatch, offsets):
         inputs.prepare_inputs_from_arrays(np.zeros(8, dtype=np.int32), np.asarray(offsets),
                                           np.full(n, 2), np.ones(n, dtype=np.int32),
                                           np.zeros(n, dtype=np.int64), "cpu")
+
+
+class _OnGpu:
+    """A CPU tensor that says it is on the first GPU."""
+
+    is_cuda = True
+    device = torch.device("cuda", 0)
+
+    def __init__(self, t):
+        self._t = t
+
+    def __getattr__(self, name):
+        return getattr(self._t, name)
+
+
+class _Library:
+    """Stands in for the two kernels of an attention call: notes who writes
+    the workspace first and who merges from it later."""
+
+    def __init__(self):
+        self.writer = {}
+        self.mixed = 0
+
+    def aegkv_paged_decode_attention_workspace_size(self, batch, *_):
+        return 1024 * batch
+
+    def aegkv_paged_decode_attention(self, *args):
+        ws, nbytes, stream = args[-3:]
+        me = threading.get_ident()
+        assert ws and nbytes == 1024 * args[11]
+        self.writer[stream, ws] = me
+        time.sleep(0.002)  # the interpreter runs other threads, as it does in a foreign call
+        self.mixed += self.writer[stream, ws] != me
+        return 0
+
+
+@pytest.mark.parametrize("streams", [[7, 7], [7, 8], [7, 7, 8, 7]])
+def test_threads_share_a_streams_workspace_in_turn(monkeypatch, streams):
+    """Two threads' calls on one stream both write the stream's workspace and
+    merge from it: a call's two kernels are enqueued with no other's between,
+    whatever the batch (the workspace grows); on two streams each has its
+    own."""
+    lib = _Library()
+    local = threading.local()
+    monkeypatch.setattr(A._lib, "load", lambda: lib)
+    monkeypatch.setattr(A, "device_guard", lambda d: nullcontext())
+    monkeypatch.setattr(A, "raw_stream", lambda d: local.stream)
+    empty = torch.empty
+    monkeypatch.setattr(A.torch, "empty", lambda *a, **k: _OnGpu(empty(*a, dtype=k["dtype"])))
+    monkeypatch.setattr(A, "_workspaces", {})
+    errors = []
+
+    def work(stream, batch):
+        local.stream = stream
+        try:
+            q = _OnGpu(torch.zeros(batch, 4, 64, dtype=torch.float16))
+            cache = _OnGpu(torch.zeros(2, 16, 1, 64, dtype=torch.float16))
+            bt = _OnGpu(torch.zeros(batch, 1, dtype=torch.int32))
+            sl = _OnGpu(torch.ones(batch, dtype=torch.int32))
+            for _ in range(20):
+                A.paged_decode_attention(q, cache, cache, bt, sl, 0.1, 16, out=q)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(s, 1 + i)) for i, s in enumerate(streams)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    assert lib.mixed == 0
+    assert len(A._workspaces) == len(set(streams))
