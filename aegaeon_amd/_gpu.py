@@ -9,6 +9,9 @@ from contextlib import nullcontext
 import torch
 
 _CURRENT = nullcontext()
+# torch's own accessor behind its stream object; not part of its documented
+# interface, so the object stands in where it is missing
+_torch_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
 
 
 def device_guard(device: torch.device):
@@ -22,6 +25,7 @@ def device_guard(device: torch.device):
 
 def raw_stream(device: torch.device) -> int:
     """The ``hipStream_t`` of torch's current stream on ``device``."""
+    if _torch_raw_stream is None:
+        return torch.cuda.current_stream(device).cuda_stream
     index = device.index
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None
-                                              else index)
+    return _torch_raw_stream(torch.cuda.current_device() if index is None else index)

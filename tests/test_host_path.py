@@ -3,6 +3,7 @@ library where a call would enqueue, are stood in for)."""
 import threading
 import time
 from contextlib import nullcontext
+from types import SimpleNamespace
 
 import numpy as np
 import pytest
@@ -33,6 +34,18 @@ def test_guard_of_the_current_gpu_switches_nothing(monkeypatch):
     _gpu.device_guard(torch.device("cuda", 0))
     _gpu.device_guard(torch.device("cuda"))
     assert switched == [torch.device("cuda", 0), torch.device("cuda")]
+
+
+def test_raw_stream_with_and_without_torchs_accessor(monkeypatch):
+    streams = {0: 70, 1: 71}
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 1)
+    monkeypatch.setattr(_gpu, "_torch_raw_stream", lambda i: streams[i])
+    devices = [torch.device("cuda", 0), torch.device("cuda", 1), torch.device("cuda")]
+    assert [_gpu.raw_stream(d) for d in devices] == [70, 71, 71]
+    monkeypatch.setattr(_gpu, "_torch_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: SimpleNamespace(
+        cuda_stream=streams[1 if d.index is None else d.index]))
+    assert [_gpu.raw_stream(d) for d in devices] == [70, 71, 71]
 
 
 @pytest.mark.parametrize("offsets", [[0, -1], [0, -2], [0, -40], [0, 3, 2], [0, 4, 1, 0]])
