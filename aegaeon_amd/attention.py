@@ -24,7 +24,7 @@ from typing import Dict, Optional, Sequence, Tuple
 import torch
 
 from . import _lib
-from ._gpu import device_guard, raw_stream
+from ._gpu import StreamBuffer, device_guard, raw_stream, stream_buffer
 
 _DTYPES = {torch.bfloat16: _lib.AEGKV_DTYPE_BF16, torch.float16: _lib.AEGKV_DTYPE_FP16}
 
@@ -218,32 +218,9 @@ def attention_workspace(batch: int, n_q_heads: int, n_kv_heads: int, head_dim: i
     return torch.empty(n, dtype=torch.uint8, device=dev)
 
 
-class _StreamWorkspace:
-    """The workspace of the calls on one stream that bring none.  A call
-    enqueues a kernel that fills it and one that merges from it, and a second
-    host thread on the stream (torch's default stream is every thread's) must
-    not come between them: ``lock`` is held while a call enqueues."""
-
-    def __init__(self):
-        self.lock = threading.Lock()
-        self.buffer: Optional[torch.Tensor] = None
-
-    def at_least(self, nbytes: int, device: torch.device) -> torch.Tensor:
-        """The buffer, grown to ``nbytes`` (lock held)."""
-        if self.buffer is None or self.buffer.numel() < nbytes:
-            self.buffer = torch.empty(nbytes, dtype=torch.uint8, device=device)
-        return self.buffer
-
-
-_workspaces: Dict[Tuple[int, int], _StreamWorkspace] = {}
+# The workspaces of the calls that bring none, one per (device, stream).
+_workspaces: Dict[Tuple[int, int], StreamBuffer] = {}
 _OWN_WORKSPACE = nullcontext()
-
-
-def _stream_workspace(device: torch.device, stream: int) -> _StreamWorkspace:
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
-    ws = _workspaces.get(key)
-    # setdefault: of threads that come here together one's entry is everyone's
-    return ws if ws is not None else _workspaces.setdefault(key, _StreamWorkspace())
 
 
 def _int32_dense(t: torch.Tensor) -> torch.Tensor:
@@ -388,7 +365,7 @@ def paged_decode_attention(q: torch.Tensor, key_cache: torch.Tensor, value_cache
         stream = raw_stream(dev)
         shared = None  # the stream's workspace when the call brings none
         if ws_bytes > 0 and workspace is None:
-            shared = _stream_workspace(dev, stream)
+            shared = stream_buffer(_workspaces, dev, stream)
         elif ws_bytes > 0:
             _check_on(workspace, "workspace", dev)
             if workspace.numel() * workspace.element_size() < ws_bytes:

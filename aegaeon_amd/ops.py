@@ -17,13 +17,14 @@ from __future__ import annotations
 
 import ctypes
 import os
-import threading
+from contextlib import nullcontext
 from typing import Dict, Optional, Sequence, Tuple, Union
 
 import numpy as np
 import torch
 
 from . import _lib
+from ._gpu import StreamBuffer, stream_buffer
 
 IdList = Union[Sequence[int], np.ndarray, torch.Tensor]
 
@@ -32,8 +33,7 @@ IdList = Union[Sequence[int], np.ndarray, torch.Tensor]
 # streams run concurrently and must not share it).
 STAGING_BYTES = int(os.environ.get("AEGKV_SWAP_STAGING_MB", "256")) << 20
 
-_staging: Dict[Tuple[int, int], torch.Tensor] = {}
-_staging_lock = threading.Lock()
+_staging: Dict[Tuple[int, int], StreamBuffer] = {}
 
 
 def _ids(x: Optional[IdList]) -> Tuple[Optional[np.ndarray], int]:
@@ -75,16 +75,6 @@ def _num_blocks(pool: torch.Tensor, bb: int) -> int:
     return pool.numel() * pool.element_size() // bb
 
 
-def _staging_for(device: torch.device, stream: int, need: int) -> torch.Tensor:
-    key = (device.index if device.index is not None else torch.cuda.current_device(), stream)
-    with _staging_lock:
-        buf = _staging.get(key)
-        if buf is None or buf.numel() < need:
-            buf = torch.empty(max(need, STAGING_BYTES), dtype=torch.uint8, device=device)
-            _staging[key] = buf
-        return buf
-
-
 def swap(source_block_ids: IdList, target_block_ids: IdList, is_swap_in: bool,
          kv_cache: torch.Tensor, kv_swap: torch.Tensor,
          staging: Union[None, str, torch.Tensor] = "auto",
@@ -103,7 +93,8 @@ def swap(source_block_ids: IdList, target_block_ids: IdList, is_swap_in: bool,
     ``staging``: "auto" packs scattered GPU blocks through a per-stream device
     buffer so that each run of consecutive CPU ids is a single DMA; None issues
     one DMA per run of consecutive id pairs; a GPU uint8 tensor is used as the
-    staging buffer directly.  The bounced path always stages.
+    staging buffer directly (by one thread at a time; the per-stream one is
+    shared by the stream's threads).  The bounced path always stages.
     """
     _require_device(kv_cache, "kv_cache")
     if kv_swap.is_cuda or not kv_swap.is_contiguous():
@@ -131,23 +122,27 @@ def swap(source_block_ids: IdList, target_block_ids: IdList, is_swap_in: bool,
         if isinstance(staging, str):
             if staging != "auto":
                 raise ValueError("staging must be 'auto', None or a tensor")
-            stg = _staging_for(device, stream, bb)
+            stg, shared = None, stream_buffer(_staging, device, stream)
         else:
-            stg = staging
+            stg, shared = staging, None
             if stg is not None and (not stg.is_cuda or stg.device != device):
                 raise ValueError(f"staging must be a GPU tensor on {device}")
-        if bounce is not None and not pinned and stg is None:
-            stg = _staging_for(device, stream, bb)
-        stg_ptr, stg_bytes = (None, 0) if stg is None else (stg.data_ptr(), stg.numel() * stg.element_size())
-        if pinned:
-            rc = _lib.load().aegkv_swap_blocks(
-                _ptr(src), _ptr(dst), n, 1 if is_swap_in else 0, kv_cache.data_ptr(), n_dev,
-                kv_swap.data_ptr(), n_host, bb, stg_ptr, stg_bytes, stream)
-        else:
-            rc = _lib.load().aegkv_swap_blocks_bounced(
-                _ptr(src), _ptr(dst), n, 1 if is_swap_in else 0, kv_cache.data_ptr(), n_dev,
-                kv_swap.data_ptr(), n_host, bb, stg_ptr, stg_bytes, bounce.data_ptr(),
-                bounce.numel() * bounce.element_size(), stream)
+            if bounce is not None and not pinned and stg is None:
+                shared = stream_buffer(_staging, device, stream)
+        with nullcontext() if shared is None else shared.lock:
+            if shared is not None:
+                stg = shared.at_least(max(bb, STAGING_BYTES), device)
+            stg_ptr, stg_bytes = (None, 0) if stg is None else \
+                (stg.data_ptr(), stg.numel() * stg.element_size())
+            if pinned:
+                rc = _lib.load().aegkv_swap_blocks(
+                    _ptr(src), _ptr(dst), n, 1 if is_swap_in else 0, kv_cache.data_ptr(), n_dev,
+                    kv_swap.data_ptr(), n_host, bb, stg_ptr, stg_bytes, stream)
+            else:
+                rc = _lib.load().aegkv_swap_blocks_bounced(
+                    _ptr(src), _ptr(dst), n, 1 if is_swap_in else 0, kv_cache.data_ptr(), n_dev,
+                    kv_swap.data_ptr(), n_host, bb, stg_ptr, stg_bytes, bounce.data_ptr(),
+                    bounce.numel() * bounce.element_size(), stream)
     _lib.check(rc, "swap")
 
 

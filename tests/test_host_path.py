@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 import torch
 
-from aegaeon_amd import _gpu, inputs
+from aegaeon_amd import _gpu, inputs, ops
 from aegaeon_amd import attention as A
 from aegaeon_amd._lib import AegkvError
 
@@ -75,8 +75,8 @@ class _OnGpu:
 
 
 class _Library:
-    """Stands in for the two kernels of an attention call: notes who writes
-    the workspace first and who merges from it later."""
+    """Stands in for the two parts of a call that shares its stream's buffer:
+    notes who fills the buffer first and who reads it later."""
 
     def __init__(self):
         self.writer = {}
@@ -86,9 +86,16 @@ class _Library:
         return 1024 * batch
 
     def aegkv_paged_decode_attention(self, *args):
-        ws, nbytes, stream = args[-3:]
+        assert args[-2] == 1024 * args[11]
+        return self._two_parts(*args[-3:])
+
+    def aegkv_swap_blocks(self, *args):
+        assert args[-2] >= args[-4]
+        return self._two_parts(*args[-3:])
+
+    def _two_parts(self, ws, nbytes, stream):
         me = threading.get_ident()
-        assert ws and nbytes == 1024 * args[11]
+        assert ws and nbytes
         self.writer[stream, ws] = me
         time.sleep(0.002)  # the interpreter runs other threads, as it does in a foreign call
         self.mixed += self.writer[stream, ws] != me
@@ -107,7 +114,7 @@ def test_threads_share_a_streams_workspace_in_turn(monkeypatch, streams):
     monkeypatch.setattr(A, "device_guard", lambda d: nullcontext())
     monkeypatch.setattr(A, "raw_stream", lambda d: local.stream)
     empty = torch.empty
-    monkeypatch.setattr(A.torch, "empty", lambda *a, **k: _OnGpu(empty(*a, dtype=k["dtype"])))
+    monkeypatch.setattr(_gpu.torch, "empty", lambda *a, **k: _OnGpu(empty(*a, dtype=k["dtype"])))
     monkeypatch.setattr(A, "_workspaces", {})
     errors = []
 
@@ -131,3 +138,40 @@ def test_threads_share_a_streams_workspace_in_turn(monkeypatch, streams):
     assert not errors, errors
     assert lib.mixed == 0
     assert len(A._workspaces) == len(set(streams))
+
+
+@pytest.mark.parametrize("staging", ["auto", None])
+def test_threads_share_a_streams_swap_staging_in_turn(monkeypatch, staging):
+    """The same for a swap's pack and its copy to the host (without staging
+    nothing is shared, and nothing is passed on)."""
+    lib = _Library()
+    if staging is None:
+        lib._two_parts = lambda ws, nbytes, stream: int(ws is not None or nbytes != 0)
+        lib.aegkv_swap_blocks = lambda *args: lib._two_parts(*args[-3:])
+    monkeypatch.setattr(ops._lib, "load", lambda: lib)
+    monkeypatch.setattr(torch.cuda, "device", lambda d: nullcontext())
+    monkeypatch.setattr(ops, "_stream", lambda d: 7)
+    monkeypatch.setattr(ops, "STAGING_BYTES", 1 << 12)
+    empty = torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, **k: _OnGpu(empty(*a, dtype=k["dtype"])))
+    monkeypatch.setattr(ops, "_staging", {})
+    errors = []
+
+    def work(width):
+        try:
+            cache = _OnGpu(torch.zeros(4, width, dtype=torch.float16))
+            host = torch.zeros(4, width, dtype=torch.float16)
+            host.is_pinned = lambda: True
+            for _ in range(20):
+                ops.swap([0, 2], [1, 3], False, cache, host, staging=staging)
+        except Exception as e:  # noqa: BLE001
+            errors.append(e)
+
+    threads = [threading.Thread(target=work, args=(w,)) for w in (64, 1 << 13)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    assert lib.mixed == 0
+    assert len(ops._staging) == (0 if staging is None else 1)
