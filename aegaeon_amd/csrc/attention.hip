@@ -148,7 +148,9 @@ inline int heads_per_group(int32_t n_kv_heads, int32_t n_wg) {
 // 1000 tokens each: 8/1 heads of 128, 32 sequences: one range 12.5 us,
 // four 14.6; 64: 16.8, two 13.9, four 15.7; 96: two 16.8, four 18.0; 192: one
 // 34.5, four 24.8.  14/2 heads of 128, 48: one 16.6, two 17.7; 128: 28.2 and
-// 28.6; 256: 47.4 and 47.2, of 64, 400: 84 and 53.
+// 28.6; 256: 47.4 and 47.2; 2/2 heads of 64, 600: 84 and 53.  (Unplanned and
+// appending calls of dim 256 do not gain: 8/2 heads, 192 sequences 75 and 79,
+// planned 81 and 77; the plan does not know the dim.)
 struct RangeRule {
   int32_t n_wg, least;  // ranges per step, and always in use
   int64_t join[3];      // positions from which 2, 3 and 4 per workgroup are
@@ -1022,8 +1024,6 @@ __device__ __forceinline__ void scan_batch(const int32_t* seq_lens, int batch, i
   }
 }
 
-// Workgroup that holds position P of the flattened range (the largest w with
-// floor(w * total / n_act) <= P; n_act <= total, so every range is non-empty).
 // floor(num / den) for 0 <= num, den < 2^52 (the host bounds every operand
 // below by that): the correctly rounded double quotient is within one of the
 // exact one, and one integer step corrects it.  A fraction of the cost of a
@@ -1036,6 +1036,8 @@ __device__ __forceinline__ int64_t div_floor(int64_t num, int64_t den) {
   return q;
 }
 
+// Range that holds position P (the largest w with floor(w * total / n_act) <= P;
+// n_act <= total, so every range is non-empty).
 __device__ __forceinline__ int64_t owner_of(int64_t P, int64_t total, int64_t n_act) {
   return div_floor((P + 1) * n_act - 1, total);
 }
