@@ -195,9 +195,10 @@ def test_deterministic(lens, heads, causal):
     """Repeated calls give the same bits (the register exchange between the
     wave halves included, also where two workgroups share a CU and their
     softmax waves a SIMD), and so does the other kernel on the same prompts
-    (a host bound of 1536 or 2048).  The ragged four-wave batch deals its
-    units round-robin over the XCDs, the co-residency under which scores read
-    before their MFMAs finished once gave run-to-run differences."""
+    (a host bound of 1536 or 2048).  The ragged four-wave batches put waves of
+    different prompts beside each other on a SIMD, the co-residency under which
+    scores read before their MFMAs finished once gave run-to-run
+    differences."""
     Hq, Hkv, D = heads
     cu, q, k, v = _packed(lens, Hq, Hkv, D, torch.bfloat16, 12)
     cu_t = torch.from_numpy(cu).cuda()
@@ -224,11 +225,11 @@ def test_qwen_prompt_batch_full_size():
 
 
 def test_units_split_into_slices_over_xcds():
-    """92 (prompt, head) units of up to 1536 tokens on the four-wave kernel:
-    92 is not a multiple of the eight XCDs and each CU has several tiles, so
-    every unit's tiles are dealt as two interleaved slices.  The output
-    matches the oracle, and equals the ping-pong kernel's (a loose bound,
-    whole units per XCD) bit for bit."""
+    """23 ragged prompts of up to 1536 tokens of four heads over one kv head,
+    on the four-wave kernel: 23 pairs, no multiple of the eight XCDs, whose
+    tiles are numbered over those that exist and fall on all XCDs.  The output
+    matches the oracle, and equals the ping-pong kernel's (a loose bound, other
+    tiles) bit for bit."""
     rng = np.random.default_rng(23)
     lens = rng.integers(1100, 1537, 23).tolist()
     lens[5] = 1536
@@ -355,8 +356,10 @@ def test_job_search_sequence_counts(n, Hq, Hkv):
 @pytest.mark.parametrize("causal", [True, False])
 @pytest.mark.parametrize("sign", [1.0, -1.0])
 def test_first_tile_sets_the_maximum(top, causal, sign):
-    """Scores that rise (or fall) by hundreds from the first key tile to the
-    later ones: the maximum the first tile sets is overtaken (or stands)."""
+    """Scores that rise (or fall) by about 3 from one key tile to the next, so
+    by 10 over 200 tokens and 77 over 1600 (a rescale waits for 8 in log2 units,
+    5.5): the maximum the first tile sets is overtaken several times (or
+    stands)."""
     lens = [top, 64, 65, 1, 129]
     cu, q, k, v = _packed(lens, 4, 2, 128, torch.float16, 31)
     for b, n in enumerate(lens):
