@@ -379,12 +379,13 @@ int aegkv_prepare_inputs(const int32_t* block_ids, const int64_t* table_offsets,
  * max_seqlen = max_prefill_seq_len (worker.py:652-711).  q [total, Hq, D],
  * k and v [total, Hkv, D], out [total, Hq, D] (DEVICE, 16-bit, token strides
  * in elements, the heads of a token contiguous, 16-byte aligned).  Sequence b
- * holds tokens [cu_seqlens[b], cu_seqlens[b+1]) (DEVICE int32 [batch + 1]);
- * query i of a sequence attends to keys j <= i of it (every key when causal
- * is 0), softmax(scale * q.k) in fp32 with P rounded to 16 bits before P.V
- * (any finite scale).  Lengths are clamped to max_seqlen (the host bound that
- * sizes the grid) and tokens to [0, total_tokens).  head_dim 64 or 128, Hq a
- * multiple of Hkv. */
+ * holds tokens [cu_seqlens[b], cu_seqlens[b+1]) (DEVICE int32 [batch + 1], not
+ * decreasing: the grid counts on sequences that share no tokens); query i of a
+ * sequence attends to keys j <= i of it (every key when causal is 0),
+ * softmax(scale * q.k) in fp32 with P rounded to 16 bits before P.V (any finite
+ * scale).  Lengths are clamped to max_seqlen (the host bound that sizes the
+ * grid) and tokens to [0, total_tokens).  head_dim 64 or 128, Hq a multiple of
+ * Hkv. */
 int aegkv_varlen_prefill_attention(void* out, int64_t out_token_stride, const void* q,
                                    int64_t q_token_stride, const void* k, int64_t k_token_stride,
                                    const void* v, int64_t v_token_stride,
