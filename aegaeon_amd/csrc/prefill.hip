@@ -69,8 +69,8 @@
 // heads: eighths 1189 us, in turn 418; unsorted 472 and 429; of one length 341
 // and 349).
 //
-// Times in this file's comments are before and after in one process on one box;
-// boxes differ by up to 4%, and the first 20 ms after a pause run slower.
+// Times in this file's comments are before and after in one process on one GPU;
+// GPUs differ by up to 4%, and the first 20 ms after a pause run slower.
 #include <algorithm>
 #include <cmath>
 

@@ -275,7 +275,7 @@ def bench_attention(args, timer, wb=None, label="Qwen2.5-7B"):
     del unplanned_out, two_out
     steps = max(g.n_layers, (args.steps // g.n_layers) * g.n_layers)
     # the five forms alternate over seven rounds and each keeps its best round,
-    # so that a slow stretch of the box does not fall on one form only
+    # so that a slow stretch of the machine does not fall on one form only
     best = {}
     for _ in range(7):
         for name, fn in (("unplanned", layer_call), ("planned", planned_call),
