@@ -105,8 +105,8 @@ constexpr int pipeline_depth() { return D >= 256 ? 2 : 3; }
 // kv heads of a workgroup's group, one per wave; the 4 / heads waves of each
 // head take ranges of their own.  Four, unless that leaves one wave in 20 or
 // more without a head; then the largest of 2 and 1 that divides the kv heads.
-// Groups of four against smaller ones, us per layer of a full chip (the kv
-// bytes of 80,000-400,000 tokens), head dim 128 and 64:
+// Groups of four against smaller ones, us per layer of a full chip (600 sequences
+// of 1000 tokens for 2 heads, 19 for 63, others between), head dim 128 and 64:
 //   kv heads      1          2          3          5          6          7
 //   128       46.5 30.1  103.2 95.2  38.5 39.5  64.7 49.9  65.5 56.8  46.6 44.0
 //   64        22.8 14.5   83.4 53.4  62.9 55.7  45.2 34.6  45.5 39.0  47.7 45.0
